@@ -659,7 +659,7 @@ def main() -> int:
         out["map_forms"] = {map_name(fmt, other): resident_batch(refs, w, h, fmt, sec_steps, 1, args.chunks,
                                                                  persistent=args.persistent, map_form=other)}
         log(f"map forms: {out['map_forms']}")
-        # Both scale strip widths (one or two output columns per lane) in
+        # Both scale strip widths (one or two 64-column waves a strip) in
         # both map forms, at the batch's default strip height.
         out["strip_widths"] = {
             f"{map_name(fmt, m)}_{cols}": resident_batch(refs, w, h, fmt, sec_steps, 1, args.chunks,

@@ -478,12 +478,10 @@ typedef struct vqm_ss2_tune_result {
 /* Times every (strip height 16/32/64/128/192/256) x (strip width 64/128) x
  * (chunks 1/2/4/8) shape for a launch of `pairs` pairs of this geometry and
  * format (rounded up to a power of two, at most 512) on the device and
- * returns the fastest; the choice is cached for the process. The strip width
- * sets the scale kernel's registers per lane and so its waves per SIMD (two
- * columns per lane: 2 waves in the reference form, 3 in the difference
- * form; one column: more). Shapes change only the order in which the FP64
- * partial sums of the strips are added (every pixel's map value and every
- * FP32 block sum is the same), so results agree to about 1e-15 relative.
+ * returns the fastest; the choice is cached for the process. Shapes change
+ * only the order in which the FP64 partial sums of the strips are added
+ * (every pixel's map value and every FP32 block sum is the same), so results
+ * agree to about 1e-15 relative.
  * Holds up to 16 GiB of temporary device memory while it runs. */
 int vqm_ss2_autotune(uint32_t width, uint32_t height, uint32_t plane_format, uint32_t map_form,
                      uint32_t pairs, vqm_ss2_tune_result* result);

@@ -1,0 +1,23 @@
+"""Builds and runs tests/cpp/row_parts_test.cc (host only): the scale kernel's
+parts tile every stored plane once and stay inside their buffers."""
+from __future__ import annotations
+
+import os
+import subprocess
+import tempfile
+
+from conftest import ROOT
+
+
+def test_row_parts():
+    with tempfile.TemporaryDirectory() as tmp:
+        exe = os.path.join(tmp, "row_parts_test")
+        subprocess.run(["g++", "-std=c++20", "-O1", "-Wall",
+                        "-I", os.path.join(ROOT, "include"),
+                        "-I", os.path.join(ROOT, "vqm_amd", "csrc"),
+                        os.path.join(ROOT, "tests", "cpp", "row_parts_test.cc"),
+                        os.path.join(ROOT, "vqm_amd", "csrc", "ss2_host.cc"),
+                        os.path.join(ROOT, "vqm_amd", "csrc", "ss2_source.cc"),
+                        "-o", exe], check=True)
+        r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stderr

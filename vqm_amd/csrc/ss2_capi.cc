@@ -220,7 +220,8 @@ int vqm_ss2_memory_plan(const vqm_ss2_config* config, vqm_ss2_memory* plan) {
         const auto g = vqm::ss2::BuildPlan(
             config->width, config->height, fmt,
             vqm::ss2::SinglePairStripRows(config->width, config->height, fmt, config->strip_rows, config->strip_cols),
-            config->strip_cols);
+            config->strip_cols,
+            vqm::ss2::SinglePairRowParts(config->width, config->height, fmt, config->strip_rows, config->strip_cols));
         const auto layout = vqm::ss2::LayoutWorkspace(g);
         vqm_image_format f;
         vqm_image_format_srgb8(&f);

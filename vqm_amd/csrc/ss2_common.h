@@ -25,9 +25,9 @@ inline constexpr int kNorms = 108;          // 18 per level
 inline constexpr int kRadius = 6;           // ceil(3.5 * 1.5), pipeline.cc:276
 inline constexpr int kTaps = 13;
 
-// Scale kernel geometry: one 64-lane wave per work item, one or two output
-// columns per lane (strips of 64 or 128 columns, Plan::strip_w). Planes are
-// padded for the widest strip.
+// Scale kernel geometry: work items are strips of 64 or 128 columns
+// (Plan::strip_w) by strip_h rows; a 64-lane wave takes a part of one, 64
+// columns by part_h rows. Planes are padded for the widest strip.
 inline constexpr int kStripCols = 128;
 inline constexpr uint32_t kDefaultStripCols = 128;
 constexpr bool ValidStripCols(uint32_t cols) { return cols == 64 || cols == 128; }
@@ -64,6 +64,8 @@ struct Plan {
     uint32_t levels;  // 1..6
     uint32_t strip_h; // output rows per scale work item
     uint32_t strip_w; // output columns per scale work item: 64 or 128
+    uint32_t part_h;  // output rows per part: strip_h, or a half or quarter of it
+    uint32_t part_shift; // log2 of the parts per item
     uint32_t w[kMaxScales], h[kMaxScales];
     uint32_t pitch[kMaxScales], rows[kMaxScales];  // padded plane geometry
     uint32_t mask[kMaxScales];                      // active channels, bit c

@@ -5,6 +5,7 @@
 #include "ss2_source.h"
 
 #include <algorithm>
+#include <bit>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
@@ -222,7 +223,8 @@ void PackView(const vqm_host_view& view, uint8_t* dst) {
     }
 }
 
-Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols) {
+Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
+              uint32_t row_parts) {
     const ScalePlan scales = PlanScales(width, height);
     if (strip_rows == 0) strip_rows = 64;
     if (strip_cols == 0) strip_cols = kDefaultStripCols;
@@ -237,6 +239,10 @@ Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t stri
     p.levels = scales.count;
     p.strip_h = strip_rows;
     p.strip_w = strip_cols;
+    if ((row_parts != 1 && row_parts != 2 && row_parts != 4) || strip_rows % (kSumBlockRows * row_parts) != 0)
+        Fail(VQM_INVALID_ARGUMENT, "a strip is cut into 1, 2 or 4 bands of a multiple of 8 rows");
+    p.part_h = strip_rows / row_parts;
+    p.part_shift = (strip_cols == kStripCols ? 1u : 0u) + row_parts / 2;
     p.plane_stride = static_cast<uint32_t>(Align(static_cast<uint64_t>(width) * height, 4));
     uint64_t cursor = 0;  // bytes
     for (uint32_t l = 0; l < static_cast<uint32_t>(kMaxScales); ++l) {
@@ -277,6 +283,9 @@ Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t stri
     return p;
 }
 
+// The CUs of a whole MI355X, for choices that are made without a device.
+constexpr uint32_t kWholeDeviceCUs = 256;
+
 uint32_t DefaultStripRows(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_cols,
                           uint64_t pairs, uint32_t cus) {
     const uint64_t per_cu = std::max<uint64_t>(cus, 1);
@@ -290,16 +299,54 @@ uint32_t DefaultStripRows(uint32_t width, uint32_t height, PlaneFormat format, u
     return 16;
 }
 
+uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
+                  uint64_t pairs, uint32_t cus) {
+    // Measured on an MI355X (256 CUs) at FP32 planes, reference form, over
+    // 96x64 to 4K and 1 to 200 pairs a launch, parts of 8 to 544 rows: a wave
+    // by itself takes 1.9 us a step; a SIMD completes a step of one of its
+    // waves every 0.85 us; and the last waves' steps, half overlapped, add
+    // 1.4 us each. The height this picks is within 1.5% of the fastest in
+    // each of the 19 launches.
+    constexpr double kAlone = 1.9, kShared = 0.85, kTail = 1.4;
+    constexpr uint32_t kStep = 4, kHaloSteps = 3;
+    const double simds = 4.0 * std::max(cus, 1u);
+    const Plan p = FillPlan(width, height, format, strip_rows, strip_cols);
+    uint32_t best = 1;
+    double best_us = 0.0;
+    for (uint32_t n : {1u, 2u, 4u}) {
+        if (p.strip_h % (kSumBlockRows * n) != 0) break;
+        const uint32_t rows = p.strip_h / n;
+        uint64_t steps = 0;
+        for (uint32_t l = 0; l < p.levels; ++l) {
+            const uint64_t columns = (p.w[l] + 63) / 64 * static_cast<uint64_t>(std::popcount(p.mask[l]));
+            const uint32_t rest = p.h[l] % rows;
+            steps += columns * (static_cast<uint64_t>(p.h[l] / rows) * (rows / kStep + kHaloSteps) +
+                                (rest ? (rest + kStep - 1) / kStep + kHaloSteps : 0));
+        }
+        const double chain = (std::min(rows, p.h[0]) + kStep - 1) / kStep + kHaloSteps;
+        const double us = std::max(kAlone * chain, kShared * static_cast<double>(steps) * pairs / simds + kTail * chain);
+        if (n == 1 || us < best_us) best = n, best_us = us;
+    }
+    return best;
+}
+
+uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
+                            uint32_t strip_cols) {
+    return strip_rows != 0 ? 1
+                           : RowParts(width, height, format,
+                                      SinglePairStripRows(width, height, format, 0, strip_cols), strip_cols, 1,
+                                      kWholeDeviceCUs);
+}
+
 uint32_t SinglePairStripRows(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                              uint32_t strip_cols) {
-    constexpr uint32_t kWholeDeviceCUs = 256;
     return strip_rows != 0 ? strip_rows : DefaultStripRows(width, height, format, strip_cols, 1, kWholeDeviceCUs);
 }
 
 GeometryPlan BuildPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
-                       uint32_t strip_cols) {
+                       uint32_t strip_cols, uint32_t row_parts) {
     GeometryPlan g;
-    g.plan = FillPlan(width, height, format, strip_rows, strip_cols);
+    g.plan = FillPlan(width, height, format, strip_rows, strip_cols, row_parts);
     g.format = format;
     g.plane_bytes_per_image = g.plan.image_bytes;
     g.prep_tiles = g.plan.prep_tiles_x * g.plan.prep_tiles_y;
@@ -311,7 +358,7 @@ GeometryPlan BuildPlan(uint32_t width, uint32_t height, PlaneFormat format, uint
 WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan) {
     WorkspaceLayout l;
     l.planes = Align(2 * plan.plane_bytes_per_image, 256);
-    l.partials = Align(static_cast<uint64_t>(std::max(plan.plan.items, 1u)) * 6 * sizeof(double), 256);
+    l.partials = Align((static_cast<uint64_t>(std::max(plan.plan.items, 1u)) << plan.plan.part_shift) * 6 * sizeof(double), 256);
     l.norms = Align(kNorms * sizeof(double), 256);
     l.total = l.planes + l.partials + l.norms;
     return l;

@@ -75,18 +75,20 @@ struct GeometryPlan {
     uint64_t plane_bytes_per_image = 0;  // padded plane storage
     PlaneFormat format = kPlaneF32;
     uint32_t prep_tiles = 0;             // prepare blocks per image
+    uint32_t parts() const { return plan.items << plan.part_shift; }  // scale blocks per pair
 };
 
 // strip_rows: output rows per scale work item, a multiple of 8 up to 1024
 // (0 = 64; launches pick theirs with DefaultStripRows); strip_cols: its
-// width, 64 or 128 columns (0 = 128).
+// width, 64 or 128 columns (0 = 128); row_parts: 1, 2 or 4 bands of a
+// multiple of 8 rows a strip is cut into, one wave each (RowParts).
 GeometryPlan BuildPlan(uint32_t width, uint32_t height, PlaneFormat format,
-                       uint32_t strip_rows, uint32_t strip_cols = 0);
+                       uint32_t strip_rows, uint32_t strip_cols = 0, uint32_t row_parts = 1);
 
 // The plan alone, without the item table (ItemAt enumerates the items):
 // nothing is allocated.
 Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
-              uint32_t strip_cols = 0);
+              uint32_t strip_cols = 0, uint32_t row_parts = 1);
 
 // The default strip height of a scale launch over `pairs` pairs of this
 // geometry on a device of `cus` compute units: 192 rows when their work
@@ -105,6 +107,20 @@ uint32_t DefaultStripRows(uint32_t width, uint32_t height, PlaneFormat format, u
 // 4K).
 uint32_t SinglePairStripRows(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                              uint32_t strip_cols);
+
+// The bands a default strip height is cut into (1, 2 or 4), by the scale
+// launch's modelled time on a device of `cus` compute units: a wave takes a
+// band in steps of four rows, three of them for the 12 halo rows, so short
+// bands repeat more work and tall ones leave a small launch waiting for one
+// wave's chain of steps. An explicit height is one band, so that equal
+// heights give equal sums whatever the launch.
+uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
+                  uint64_t pairs, uint32_t cus);
+
+// RowParts of a single-pair pipeline's default height (of the geometry
+// alone, as SinglePairStripRows); 1 when `strip_rows` is set.
+uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
+                            uint32_t strip_cols);
 
 // Bytes of one pair's workspace: planes of both images, partials, norms,
 // each rounded to 256 bytes.

@@ -10,7 +10,7 @@
 namespace vqm::ss2 {
 
 // A flat work list entry: pair index in the batch and the local work index
-// (prepare: tile | image << 31; scale: item). Used when a batch mixes
+// (prepare: tile | image << 31; scale: part). Used when a batch mixes
 // geometries; a batch of one geometry indexes blocks arithmetically.
 struct WorkRef {
     uint32_t pair;
@@ -33,16 +33,14 @@ hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const Pa
                          const uint8_t* src0, const uint8_t* src1, hipStream_t stream,
                          bool persistent = false);
 
-// One 64-lane wave per scale work item (level, channel, strip of 64 or 128
-// columns). Uniform geometry: blocks = pairs * items_per_pair, work =
-// nullptr. `blur` picks the kernel: kBlurSampled (13-tap sampled Gaussian)
+// One 64-lane wave per part of a scale work item (level, channel, 64 columns
+// by Plan::part_h rows). Uniform geometry: blocks = pairs * parts_per_pair,
+// work = nullptr; else work[].index is a part. `blur` picks the kernel: kBlurSampled (13-tap sampled Gaussian)
 // or kBlurRecursive (the recursive Gaussian's 9-tap truncated-cosine
 // kernel); `map` the SSIM' map's form, which must be the one the planes were
-// prepared with; `strip_cols` the strip width of every plan in the launch
-// (Plan::strip_w).
-hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, uint32_t strip_cols,
-                       const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t items_per_pair,
-                       hipStream_t stream, bool persistent = false);
+// prepared with.
+hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
+                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent = false);
 
 // Sums each (level, channel) norm's partials in FP64 and writes the 108 norms.
 hipError_t LaunchReduce(const PairDesc* pairs, uint32_t pairs_count, hipStream_t stream);

@@ -3,14 +3,14 @@
 //   prepare  u8 sRGB -> linear (256-entry table) -> XYB, plus the 2x2 box
 //            pyramid of the linear planes, writing only the (level, channel)
 //            planes whose maps survive pruning (prepare.comp:170-232).
-//   scale    one wave per strip (128 or 64 columns) of one (level,
-//            channel): the 13-tap blurs of the map's quantities, the SSIM'
-//            and edge maps, and six map sums, FP32 over 8-row blocks then
-//            FP64 (scale.comp:335-437). Rows stream through the wave: each
-//            input row is staged in LDS, blurred horizontally (each lane owns
-//            two output columns, or one), and the horizontal results enter a
-//            13-row register ring from which the vertical blur of the row six
-//            above is taken. No map ever reaches HBM.
+//   scale    one wave per 64-column part of a strip of one (level, channel):
+//            the 13-tap blurs of the map's quantities, the SSIM' and edge
+//            maps, and six map sums, FP32 over 8-row blocks then FP64
+//            (scale.comp:335-437). Rows stream through the wave four at a
+//            time: staged in LDS, blurred horizontally (lane = row and four
+//            columns), turned in LDS to lane = column, and added to the
+//            partial sums of the output rows that wait for them. No map ever
+//            reaches HBM.
 //   reduce   FP64 sum of each norm's per-strip partials, 1-norm means and
 //            4-norm fourth roots (reduce.comp:21-63, vulkan.cc:545-583).
 //
@@ -75,6 +75,14 @@ constexpr float kC2 = 0.0009f;            // scale.comp:87
 
 __device__ __forceinline__ float fma_(float a, float b, float c) {
     return __builtin_fmaf(a, b, c);
+}
+
+// fma(w, x, c) for a constant w into a register of its own: the compiler
+// forms it in c's register and copies that away where c's name changes.
+__device__ __forceinline__ float fma_move(float w, float x, float c) {
+    float r;
+    asm("v_fmamk_f32 %0, %1, %3, %2" : "=v"(r) : "v"(x), "v"(c), "i"(__builtin_bit_cast(int, w)));
+    return r;
 }
 
 // Smallest normal float: the XYB mixes are clamped to it instead of 0, so the
@@ -222,12 +230,13 @@ __device__ __forceinline__ void xyb_group(const float (*px)[3], uint32_t mask, f
 // one row later instead of right behind the load.
 struct F32 {
     using E = float;
-    using Raw = f32x2;
-    static __device__ __forceinline__ Raw load2(GlobalAS<const E>* p) {
-        return *reinterpret_cast<GlobalAS<const f32x2>*>(p);
+    using Raw4 = f32x4;
+    static __device__ __forceinline__ Raw4 load4(GlobalAS<const E>* p) {
+        return Raw4{p[0], p[1], p[2], p[3]};
     }
-    static __device__ __forceinline__ float2 unpack(Raw v) { return make_float2(v.x, v.y); }
-    static __device__ __forceinline__ float unpack1(E v) { return v; }
+    static __device__ __forceinline__ void unpack4(Raw4 v, float out[4]) {
+        for (int i = 0; i < 4; ++i) out[i] = v[i];
+    }
     static __device__ __forceinline__ void store1(GlobalAS<E>* p, float v) { *p = v; }
     static __device__ __forceinline__ void store2(GlobalAS<E>* p, float a, float b) {
         *reinterpret_cast<GlobalAS<f32x2>*>(p) = f32x2{a, b};
@@ -267,15 +276,17 @@ __device__ __forceinline__ float from_bf16(uint16_t v) {
 template <uint16_t (*To)(float), float (*From)(uint16_t)>
 struct Narrow {
     using E = uint16_t;
-    using Raw = uint32_t;
-    static __device__ __forceinline__ Raw load2(GlobalAS<const E>* p) {
-        return *reinterpret_cast<GlobalAS<const uint32_t>*>(p);
+    using Raw4 = u32x2;
+    static __device__ __forceinline__ Raw4 load4(GlobalAS<const E>* p) {
+        GlobalAS<const uint32_t>* w = reinterpret_cast<GlobalAS<const uint32_t>*>(p);
+        return Raw4{w[0], w[1]};
     }
-    static __device__ __forceinline__ float2 unpack(Raw v) {
-        return make_float2(From(static_cast<uint16_t>(v & 0xFFFFu)),
-                           From(static_cast<uint16_t>(v >> 16)));
+    static __device__ __forceinline__ void unpack4(Raw4 v, float out[4]) {
+        for (int i = 0; i < 2; ++i) {
+            out[2 * i] = From(static_cast<uint16_t>(v[i] & 0xFFFFu));
+            out[2 * i + 1] = From(static_cast<uint16_t>(v[i] >> 16));
+        }
     }
-    static __device__ __forceinline__ float unpack1(E v) { return From(v); }
     static __device__ __forceinline__ void store1(GlobalAS<E>* p, float v) { *p = To(v); }
     static __device__ __forceinline__ void store2(GlobalAS<E>* p, float a, float b) {
         *reinterpret_cast<GlobalAS<uint32_t>*>(p) =
@@ -1023,15 +1034,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(General ? 5
 
 // ---- scale ------------------------------------------------------------------
 
-constexpr int kRing = 8;  // raw rows kept in LDS: the map needs the row six back
+// What bounds it: VALU issue and, at full rate, the clock. A SIMD issues FP32
+// adds, multiplies and fused multiply-adds of two waves at once, one per wave
+// every 4.5 cycles (5.1 with a literal operand): 2.2 to 2.6 cycles an
+// instruction from two waves up, an even number of them (three share as one
+// and two: 1.30 against 0.99 ns an instruction). Only one of the two may be a
+// min/max, a conversion, a shift or any instruction with an SGPR operand, and
+// FP64 and transcendental instructions take both (4.2 and 8.2 cycles). The
+// taps are literals: held in VGPRs the instructions read three registers and
+// the launch took 4.62 ms against 4.24 (300 1080p pairs).
+//
+// Hence four waves a SIMD, 128 registers: one column a lane, not two (a
+// 13-row ring of five quantities and two columns alone was 130). The ring is
+// kept as the partial sums of the 12 output rows that still wait for source
+// rows: a step of four rows completes four of them, and the multiply-add that
+// takes a sum's next tap also moves it four places on, so the loop needs no
+// unrolling by rows (8.7 KB of code against 45; a wave of a 96x64 pair spends
+// 17 us against 30, most of it fetching instructions). FP64 sums live in LDS,
+// 10,176 bytes a wave, sixteen waves a CU.
+//
+// Lanes take four columns of one row in the horizontal pass, so a row's 16
+// source samples serve four outputs: 16 bytes of LDS reads an output and
+// image in 16-byte accesses, and the products formed in registers, against
+// 52 bytes a quantity for a column a lane. (An LDS read of 16 bytes a lane
+// runs at 245 B/cycle a CU; the pair of 8-byte reads the two-column form
+// compiled to, at 125.)
+//
+// 300 1080p pairs, reference form: 5.45 -> 4.24 ms, 3.37e9 wave instructions
+// at 2.4 cycles each per SIMD (3.7 before), at a clock of about 1.9 GHz (2.2
+// before: the chip lowers it as the issue rate rises). 60 pairs of 640x360 to
+// 4K: 1.71 -> 1.19 ms; one 4K pair: 91 -> 75 us.
+constexpr int kStep = 4;             // source rows a wave takes per step
+constexpr int kPending = kTaps - 1;  // output rows that wait for more source rows
+constexpr int kSrcCols = 64 + 2 * kRadius;
+constexpr int kRawRows = kStep + kRadius;  // raw rows kept in LDS: the step's and the six before them
 
-// Blurred quantities and the products staged beside the raw rows, by form:
+// Blurred quantities by form:
 // the reference form blurs a, b, a*a, b*b and a*b (scale.comp:130-142); the
 // difference form a, b, (a - b)^2 and a*b.
-template <bool Ref> struct MapQuantities {
-    static constexpr int kBlurred = Ref ? 5 : 4;
-    static constexpr int kProducts = kBlurred - 2;
-};
+template <bool Ref> constexpr int kBlurred = Ref ? 5 : 4;
 
 template <int... P, typename F>
 __device__ __forceinline__ void unroll(std::integer_sequence<int, P...>, F&& f) {
@@ -1041,77 +1082,6 @@ __device__ __forceinline__ void unroll(std::integer_sequence<int, P...>, F&& f) 
 __device__ __forceinline__ double wave_sum(double v) {
     for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
     return v;
-}
-
-// Strip geometry of a scale work item: 64 lanes of Cols output columns
-// each (64- or 128-column strips), the source row wider by the blur radius
-// on both sides; the 12 halo columns are loaded by the first 12 / Cols lanes.
-template <int Cols>
-struct StripGeom {
-    static_assert(Cols == 1 || Cols == 2, "one or two output columns per lane");
-    static constexpr int kCols = 64 * Cols;
-    static constexpr int kSrc = kCols + 2 * kRadius;
-    static constexpr int kHaloLanes = 2 * kRadius / Cols;
-};
-
-// A lane's Cols adjacent plane samples of one row: loaded as raw bits,
-// unpacked to FP32 where they are consumed.
-template <typename Fmt, int Cols> struct LaneSamples;
-template <typename Fmt> struct LaneSamples<Fmt, 2> {
-    using Raw = typename Fmt::Raw;
-    static __device__ __forceinline__ Raw load(GlobalAS<const typename Fmt::E>* p) { return Fmt::load2(p); }
-    static __device__ __forceinline__ void unpack(Raw v, float out[2]) {
-        const float2 t = Fmt::unpack(v);
-        out[0] = t.x;
-        out[1] = t.y;
-    }
-};
-template <typename Fmt> struct LaneSamples<Fmt, 1> {
-    using Raw = typename Fmt::E;
-    static __device__ __forceinline__ Raw load(GlobalAS<const typename Fmt::E>* p) { return *p; }
-    static __device__ __forceinline__ void unpack(Raw v, float out[1]) { out[0] = Fmt::unpack1(v); }
-};
-
-// Cols adjacent floats to and from LDS (one 8-byte access for two).
-template <int Cols>
-__device__ __forceinline__ void lds_put(float* p, const float* v) {
-    if constexpr (Cols == 2) {
-        *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
-    } else {
-        *p = v[0];
-    }
-}
-template <int Cols>
-__device__ __forceinline__ void lds_get(const float* p, float* v) {
-    if constexpr (Cols == 2) {
-        const float2 t = *reinterpret_cast<const float2*>(p);
-        v[0] = t.x;
-        v[1] = t.y;
-    } else {
-        v[0] = *p;
-    }
-}
-
-// The products of one lane's samples of a and b that the form blurs, staged
-// at source column j of each product row.
-template <bool Ref, int Cols>
-__device__ __forceinline__ void stage_products(float (*prod)[StripGeom<Cols>::kSrc], int j, const float* a,
-                                               const float* b) {
-    float p0[Cols], p1[Cols], p2[Cols];
-    for (int c = 0; c < Cols; ++c) {
-        if constexpr (Ref) {
-            p0[c] = a[c] * a[c];
-            p1[c] = b[c] * b[c];
-            p2[c] = a[c] * b[c];
-        } else {
-            const float d = a[c] - b[c];
-            p0[c] = d * d;
-            p1[c] = a[c] * b[c];
-        }
-    }
-    lds_put<Cols>(&prod[0][j], p0);
-    lds_put<Cols>(&prod[1][j], p1);
-    if constexpr (Ref) lds_put<Cols>(&prod[2][j], p2);
 }
 
 // The six map values of one pixel from its blurred quantities `bl` (in the
@@ -1164,200 +1134,280 @@ __device__ __forceinline__ void map_values(const float* bl, float a, float b, fl
     v6[5] = bb * bb;
 }
 
-// One scale work item: the strip of `level`, `channel` starting at (x0, y0),
-// with the plane elements in format Fmt and Cols output columns per lane.
-template <typename Fmt, typename TapsT, bool Ref, int Cols>
-__device__ __forceinline__ void scale_item(ConstAS<PairDesc>* pdp, ConstAS<Plan>* plan, uint32_t item_idx,
-                                           uint32_t level, uint32_t channel, uint32_t x0, uint32_t y0,
-                                           float (*ring_a)[StripGeom<Cols>::kSrc],
-                                           float (*ring_b)[StripGeom<Cols>::kSrc],
-                                           float (*prod)[StripGeom<Cols>::kSrc]) {
-    using Geo = StripGeom<Cols>;
-    using IO = LaneSamples<Fmt, Cols>;
-    constexpr int kBlurred = MapQuantities<Ref>::kBlurred;
-    const uint32_t W = plan->w[level], H = plan->h[level], pitch = plan->pitch[level];
-    // The strip's output rows stop at the level's last row (y0 < H for every
-    // item): rows past it would be blurred and then dropped, up to half of
-    // a strip on the small levels.
-    const int total = static_cast<int>(min(plan->strip_h, H - y0)) + 2 * kRadius;
 
-    using E = typename Fmt::E;
-    // Source row r (0 .. total-1) is image row y0 - 6 + r, padded row y0 + r;
-    // source column j (0 .. kSrc-1) is image column x0 - 6 + j, padded
-    // x0 + 2 + j.
-    GlobalAS<const uint8_t>* base = as_global(static_cast<const uint8_t*>(pdp->planes));
-    GlobalAS<const E>* pa = reinterpret_cast<GlobalAS<const E>*>(base + plan->plane_off[level][channel]) +
-                            (static_cast<uint64_t>(y0) * pitch + x0 + 2u);
-    GlobalAS<const E>* pb = reinterpret_cast<GlobalAS<const E>*>(
-        reinterpret_cast<GlobalAS<const uint8_t>*>(pa) + plan->image_bytes);
-
-    const int lane = static_cast<int>(threadIdx.x);
-    const bool halo = lane < Geo::kHaloLanes;
-    const int jm = Cols * lane, jh = Geo::kCols + Cols * lane;
-
-    typename IO::Raw cur_a = IO::load(pa + jm), cur_b = IO::load(pb + jm);
-    typename IO::Raw cur_ha{}, cur_hb{};
-    if (halo) {
-        cur_ha = IO::load(pa + jh);
-        cur_hb = IO::load(pb + jh);
-    }
-
-    float win[kTaps][kBlurred][Cols];
-    // Map sums: each lane adds each of its columns' values over a block of
-    // eight rows (rows 8k .. 8k+7 of the level, in row order) in FP32, then
-    // the block's sum into FP64. Strips start on rows that are multiples of
-    // eight, so the blocks, and every FP32 sum, do not depend on the strip
-    // geometry.
-    float block[Cols][6];
-    for (int c = 0; c < Cols; ++c)
-        for (int k = 0; k < 6; ++k) block[c][k] = 0.0f;
-    double sums[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    const uint32_t col = x0 + static_cast<uint32_t>(jm);
-
-    for (int base_row = 0; base_row < total; base_row += kTaps) {
-        unroll(std::make_integer_sequence<int, kTaps>{}, [&](auto pc) {
-            constexpr int P = decltype(pc)::value;
-            const int i = base_row + P;
-            if (i >= total) return;
-            // Stage input row i: raw samples into the ring, products alongside.
-            float* ra = ring_a[i & (kRing - 1)];
-            float* rb = ring_b[i & (kRing - 1)];
-            {
-                float a[Cols], b[Cols];
-                IO::unpack(cur_a, a);
-                IO::unpack(cur_b, b);
-                lds_put<Cols>(ra + jm, a);
-                lds_put<Cols>(rb + jm, b);
-                stage_products<Ref, Cols>(prod, jm, a, b);
-            }
-            if (halo) {
-                float a[Cols], b[Cols];
-                IO::unpack(cur_ha, a);
-                IO::unpack(cur_hb, b);
-                lds_put<Cols>(ra + jh, a);
-                lds_put<Cols>(rb + jh, b);
-                stage_products<Ref, Cols>(prod, jh, a, b);
-            }
-            // Prefetch input row i + 1.
-            if (i + 1 < total) {
-                const uint64_t off = static_cast<uint64_t>(i + 1) * pitch;
-                cur_a = IO::load(pa + off + jm);
-                cur_b = IO::load(pb + off + jm);
-                if (halo) {
-                    cur_ha = IO::load(pa + off + jh);
-                    cur_hb = IO::load(pb + off + jh);
-                }
-            }
-            __syncthreads();
-
-            // Horizontal 13-tap pass of each blurred quantity at this lane's
-            // output columns (source columns jm + 6 .. jm + 5 + Cols).
-            for (int q = 0; q < kBlurred; ++q) {
-                const float* s = q == 0 ? ra : q == 1 ? rb : prod[q - 2];
-                float v[kTaps - 1 + Cols];
-                for (int k = 0; k < kTaps - 1 + Cols; k += Cols) lds_get<Cols>(s + jm + k, v + k);
-                for (int c = 0; c < Cols; ++c) {
-                    float h = TapsT::w[0] * v[c];
-                    for (int k = 1; k < kTaps; ++k) h = fma_(TapsT::w[k], v[k + c], h);
-                    win[P][q][c] = h;
-                }
-            }
-
-            // Vertical pass for output row i - 12 (image row y0 + i - 12),
-            // oldest ring entry first: scale.comp:243-298's ascending taps.
-            if (i >= 2 * kRadius) {
-                auto vertical = [&](int c, float* out) {
-                    for (int q = 0; q < kBlurred; ++q) {
-                        float acc = TapsT::w[0] * win[(P + 1) % kTaps][q][c];
-                        for (int k = 1; k < kTaps; ++k)
-                            acc = fma_(TapsT::w[k], win[(P + 1 + k) % kTaps][q][c], acc);
-                        out[q] = acc;
-                    }
-                };
-                const uint32_t y = y0 + static_cast<uint32_t>(i - 2 * kRadius);
-                const int raw_slot = (i - kRadius) & (kRing - 1);
-                float av[Cols], bv[Cols];
-                lds_get<Cols>(&ring_a[raw_slot][jm + kRadius], av);
-                lds_get<Cols>(&ring_b[raw_slot][jm + kRadius], bv);
-                if (y < H) {
-                    if constexpr (Ref) {
-                        // One column at a time: its five blurred values
-                        // live only through its map.
-                        for (int c = 0; c < Cols; ++c) {
-                            float bl[kBlurred];
-                            vertical(c, bl);
-                            if (col + static_cast<uint32_t>(c) >= W) continue;
-                            float v6[6];
-                            map_values<true>(bl, av[c], bv[c], v6);
-                            for (int k = 0; k < 6; ++k) block[c][k] = block[c][k] + v6[k];
-                        }
-                    } else {
-                        float bl[Cols][kBlurred];
-                        for (int c = 0; c < Cols; ++c) vertical(c, bl[c]);
-                        for (int c = 0; c < Cols; ++c) {
-                            if (col + static_cast<uint32_t>(c) >= W) continue;
-                            float v6[6];
-                            map_values<false>(bl[c], av[c], bv[c], v6);
-                            for (int k = 0; k < 6; ++k) block[c][k] = block[c][k] + v6[k];
-                        }
-                    }
-                    // A block ends on rows 7, 15, 23, ... and on the level's
-                    // last row (a uniform branch: y is the wave's row).
-                    if ((y & 7u) == 7u || y + 1u == H) {
-                        for (int c = 0; c < Cols; ++c)
-                            for (int k = 0; k < 6; ++k) {
-                                sums[k] += static_cast<double>(block[c][k]);
-                                block[c][k] = 0.0f;
-                            }
-                    }
-                }
-            }
-        });
-    }
-
-    GlobalAS<double>* out = as_global(pdp->partials) + static_cast<uint64_t>(item_idx) * 6u;
-    for (int k = 0; k < 6; ++k) {
-        const double s = wave_sum(sums[k]);
-        if (lane == 0) out[k] = s;
-    }
+// Orders a wave's LDS accesses: the wave's own are executed in order by the
+// hardware, so only the compiler has to keep them apart.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// Work items blockIdx.x, blockIdx.x + gridDim.x, ... of `blocks`, as in
-// prepare_kernel. Two columns per lane hold a 130-register ring in the
-// reference form (two waves per SIMD) and a 104-register one in the
-// difference form, held to 168 registers (three waves); one column per lane
-// halves the ring (four waves).
-template <int Cols, bool Ref>
-constexpr int kScaleWaves = (Cols == 2 && !Ref) ? 3 : 1;
+// One wave's LDS: the raw rows of the last kRawSlots steps, and the
+// exchange that turns horizontal results (lane = row and column group) into
+// the vertical pass's (lane = column).
+struct ScaleLds {
+    float raw[2][kRawRows][kSrcCols];
+    float turn[kStep][64];
+    double sums[6][64];
+};
 
-template <typename Lay, typename TapsT, bool Ref, int Cols>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kScaleWaves<Cols, Ref>))) void scale_kernel(const PairDesc* __restrict__ pairs,
-                                                   const WorkRef* __restrict__ work,
-                                                   uint32_t blocks, uint32_t items_per_pair) {
-    constexpr int kSrc = StripGeom<Cols>::kSrc;
-    __shared__ __align__(16) float ring_a[kRing][kSrc];
-    __shared__ __align__(16) float ring_b[kRing][kSrc];
-    __shared__ __align__(16) float prod[MapQuantities<Ref>::kProducts][kSrc];
+// One wave's part of a scale work item: 64 columns from x0 of the strip
+// whose first row is y0, with the plane elements in format Fmt. Leaves the
+// six map sums of each column in lds.sums.
+template <typename Fmt, typename TapsT, bool Ref>
+__device__ __forceinline__ void scale_strip(ConstAS<PairDesc>* pdp, ConstAS<Plan>* plan, uint32_t level,
+                                            uint32_t channel, uint32_t x0, uint32_t y0, ScaleLds& lds) {
+    using E = typename Fmt::E;
+    constexpr int Q = kBlurred<Ref>;
+    const uint32_t H = plan->h[level], pitch = plan->pitch[level];
+    // The part's output rows stop at the level's last row.
+    const int total = static_cast<int>(min(plan->part_h, H - y0)) + 2 * kRadius;
+
+    // Source row r (0 .. total-1) is image row y0 - 6 + r, padded row y0 + r;
+    // source column j (0 .. 75) is image column x0 - 6 + j, padded x0 + 2 + j.
+    GlobalAS<const uint8_t>* pa =
+        as_global(static_cast<const uint8_t*>(pdp->planes)) + plan->plane_off[level][channel] +
+        (static_cast<uint64_t>(y0) * pitch + x0 + 2u) * sizeof(E);
+    GlobalAS<const uint8_t>* pb = pa + plan->image_bytes;
+    auto load = [](GlobalAS<const uint8_t>* p, uint32_t offset) {
+        return Fmt::load4(reinterpret_cast<GlobalAS<const E>*>(p + offset));
+    };
+
+    // Horizontal roles: lane = source row `r` of the step and four columns
+    // from 4 g. The 12 halo columns of the step's rows are three quads a row
+    // and image, loaded by lanes 0 .. 11 (a) and 16 .. 27 (b).
+    uint32_t lane = threadIdx.x & 63u;
+    asm volatile("" : "+v"(lane));  // nothing formed from it is held across items
+    const uint32_t r = lane >> 4, g = lane & 15u;
+    const bool halo = g < 3u * kStep && lane < 32u;
+    const uint32_t hr = (g < 12u ? g : 0u) / 3u, hc = 64u + 4u * (g - 3u * hr);
+    const uint32_t at = (r * pitch + 4u * g) * sizeof(E), halo_at = (hr * pitch + hc) * sizeof(E);
+    float* const halo_to = &lds.raw[lane < 16u ? 0 : 1][0][hc];
+
+    const bool halo_b = lane >= 16u;
+    typename Fmt::Raw4 cur_a = load(pa, at), cur_b = load(pb, at), cur_h = load(halo_b ? pb : pa, halo_at);
+
+    // The vertical pass in flight: partial sums of the 12 output rows that
+    // still miss source rows, oldest first.
+    float part[Q][kPending];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int m = 0; m < kPending; ++m) part[q][m] = 0.0f;
+    float block[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        block[k] = 0.0f;
+        lds.sums[k][lane] = 0.0;
+    }
+    uint32_t slot = 0;  // the ring row of the step's first row
+
+    for (int i0 = 0; i0 < total; i0 += kStep) {
+        // The lane's LDS addresses are formed again each step rather than
+        // held: registers are what limits the waves in flight.
+        asm("" : "+v"(lane));
+        const uint32_t r = lane >> 4, g = lane & 15u;
+        // Stage the step's rows.
+        auto ring = [&](uint32_t row) { return row >= kRawRows ? row - kRawRows : row; };
+        float* const ra = &lds.raw[0][0][0] + (ring(slot + r) * kSrcCols + 4u * g);
+        float* const rb = ra + kRawRows * kSrcCols;
+        {
+            float v[4];
+            Fmt::unpack4(cur_a, v);
+            *reinterpret_cast<f32x4*>(ra) = f32x4{v[0], v[1], v[2], v[3]};
+            Fmt::unpack4(cur_b, v);
+            *reinterpret_cast<f32x4*>(rb) = f32x4{v[0], v[1], v[2], v[3]};
+            if (halo) {
+                Fmt::unpack4(cur_h, v);
+                *reinterpret_cast<f32x4*>(halo_to + ring(slot + hr) * kSrcCols) = f32x4{v[0], v[1], v[2], v[3]};
+            }
+        }
+        wave_fence();
+
+        // Horizontal 13-tap pass: columns 4 g .. 4 g + 3 of row r, source
+        // columns in ascending order so that every chain's taps ascend
+        // (scale.comp:187-241).
+        float acc[Q][4];
+        {
+            f32x4 va = *reinterpret_cast<const f32x4*>(ra), vb = *reinterpret_cast<const f32x4*>(rb);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                f32x4 na{}, nb{};
+                if (t < 3) {
+                    na = *reinterpret_cast<const f32x4*>(ra + 4 * t + 4);
+                    nb = *reinterpret_cast<const f32x4*>(rb + 4 * t + 4);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int m = 4 * t + e;
+                    const float x = va[e], y = vb[e];
+                    float v[Q];
+                    v[0] = x;
+                    v[1] = y;
+                    if constexpr (Ref) {
+                        v[2] = x * x;
+                        v[3] = y * y;
+                        v[4] = x * y;
+                    } else {
+                        const float d = x - y;
+                        v[2] = d * d;
+                        v[3] = x * y;
+                    }
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            const int k = m - c;
+                            if (k == 0) acc[q][c] = TapsT::w[0] * v[q];
+                            if (k > 0 && k < kTaps) acc[q][c] = fma_(TapsT::w[k], v[q], acc[q][c]);
+                        }
+                }
+                va = na;
+                vb = nb;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+
+        // The next step's rows, in flight until its start. (The last step
+        // loads its own again: the rows after it may lie past the plane. A
+        // branch around the loads lets the compiler sink the sums above past
+        // them, which spills.)
+        const uint32_t advance = i0 + kStep < total ? kStep * pitch * static_cast<uint32_t>(sizeof(E)) : 0u;
+        pa += advance;
+        pb += advance;
+        cur_a = load(pa, at);
+        cur_b = load(pb, at);
+        cur_h = load(halo_b ? pb : pa, halo_at);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // Turn each quantity's results to lane = column and add the four new
+        // rows to the pending output rows, taps ascending with the source
+        // row (scale.comp:243-298). Output rows i0 - 12 .. i0 - 9 complete.
+        float done[kStep][Q], h[2][kStep];
+        auto turn = [&](int q) {
+            *reinterpret_cast<f32x4*>(&lds.turn[0][4u * lane]) = f32x4{acc[q][0], acc[q][1], acc[q][2], acc[q][3]};
+            wave_fence();
+#pragma unroll
+            for (int j = 0; j < kStep; ++j) h[q & 1][j] = lds.turn[j][lane];
+            wave_fence();
+        };
+        turn(0);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            if (q + 1 < Q) turn(q + 1);  // in flight while this quantity's rows are added
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < kPending + kStep; ++m) {
+                // Output row i0 - 12 + m: new row j is its tap 12 - m + j.
+                float v = m < kPending ? part[q][m] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < kStep; ++j) {
+                    const int k = kTaps - 1 - m + j;
+                    if (k == 0) v = TapsT::w[0] * h[q & 1][j];
+                    if (k > 0 && k < kTaps)
+                        v = j == 0 ? fma_move(TapsT::w[k], h[q & 1][j], v) : fma_(TapsT::w[k], h[q & 1][j], v);
+                }
+                if (m < kStep) done[m][q] = v; else part[q][m - kStep] = v;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+        // The pixels' own samples: source rows i - 6, kStep rows on in the
+        // ring (nothing uses them before the first output row).
+        float own[kStep][2];
+#pragma unroll
+        for (int j = 0; j < kStep; ++j) {
+            const float* const at_j = &lds.raw[0][0][kRadius] + (ring(slot + kStep + j) * kSrcCols + lane);
+            own[j][0] = at_j[0];
+            own[j][1] = at_j[kRawRows * kSrcCols];
+        }
+        unroll(std::make_integer_sequence<int, kStep>{}, [&](auto jc) {
+            constexpr int J = decltype(jc)::value;
+            if (i0 < 2 * kRadius || i0 + J >= total) return;
+            float v6[6];
+            map_values<Ref>(done[J], own[J][0], own[J][1], v6);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) block[k] = block[k] + v6[k];
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        // Rows 8k .. 8k+7 of the level end with every second step; the
+        // level's last rows are added after the loop.
+        if ((i0 & kStep) == 0) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                lds.sums[k][lane] += static_cast<double>(block[k]);
+                block[k] = 0.0f;
+            }
+        }
+        slot = ring(slot + kStep);
+        wave_fence();
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) lds.sums[k][lane] += static_cast<double>(block[k]);
+}
+
+// v plus lane (l ^ 1)'s, (l ^ 2)'s or (7 - l % 8)'s v, by DPP control.
+template <int Ctrl>
+__device__ __forceinline__ double add_dpp(double v) {
+    const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(bits), Ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(bits >> 32), Ctrl, 0xF, 0xF, true);
+    return v + __builtin_bit_cast(double, static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32 | static_cast<uint32_t>(lo));
+}
+
+// The wave's map sums over its first `cols` columns: lanes 8 k .. 8 k + 7
+// (k < 6) return map k's, each lane adding every eighth column.
+__device__ __forceinline__ double sum_columns(const ScaleLds& lds, uint32_t lane, uint32_t cols) {
+    const uint32_t k = min(lane >> 3, 5u);
+    double v = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t c = (lane & 7u) + 8u * i;
+        v += c < cols ? lds.sums[k][c] : 0.0;
+    }
+    v = add_dpp<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+    v = add_dpp<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+    return add_dpp<0x141>(v);  // row_half_mirror
+}
+
+// Parts blockIdx.x, blockIdx.x + gridDim.x, ... of `blocks`, one wave each:
+// item * parts_per_item + sub, where an item's parts run over its 64-column
+// halves, then its part_h-row bands.
+template <typename Lay, typename TapsT, bool Ref>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void scale_kernel(
+    const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ work, uint32_t blocks, uint32_t parts_per_pair) {
+    __shared__ __align__(16) ScaleLds lds;
 
     for (uint32_t b = blockIdx.x; b < blocks; b += gridDim.x) {
-        uint32_t pair_idx, item_idx;
+        uint32_t pair_idx, part;
         if (work != nullptr) {
             ConstAS<WorkRef>* w = as_const(work) + xcd_remap(b, blocks);
             pair_idx = w->pair;
-            item_idx = w->index;
+            part = w->index;
         } else {
             const uint32_t l = xcd_remap(b, blocks);
-            pair_idx = l / items_per_pair;
-            item_idx = l % items_per_pair;
+            pair_idx = l / parts_per_pair;
+            part = l % parts_per_pair;
         }
         ConstAS<PairDesc>* pdp = as_const(pairs) + pair_idx;
         ConstAS<Plan>* plan = as_const(pdp->plan);
-        ConstAS<ScaleItem>* item = as_const(pdp->items) + item_idx;
+        const uint32_t shift = plan->part_shift, wide = plan->strip_w / 128u;
+        ConstAS<ScaleItem>* item = as_const(pdp->items) + (part >> shift);
+        const uint32_t sub = part & ((1u << shift) - 1u);
         const uint32_t level = item->level, channel = item->channel;
-        const uint32_t x0 = item->x0, y0 = item->y0;
-        scale_item<typename Lay::Fmt, TapsT, Ref, Cols>(pdp, plan, item_idx, level, channel, x0, y0, ring_a,
-                                                        ring_b, prod);
-        __syncthreads();  // the next item reuses the row ring
+        const uint32_t x0 = item->x0 + 64u * (sub & wide), y0 = item->y0 + (sub >> wide) * plan->part_h;
+        const uint32_t W = plan->w[level];
+        uint32_t lane = threadIdx.x & 63u;
+        double v = 0.0;
+        if (x0 < W && y0 < plan->h[level]) {  // else the item's strip ends before this part
+            scale_strip<typename Lay::Fmt, TapsT, Ref>(pdp, plan, level, channel, x0, y0, lds);
+            asm volatile("" : "+v"(lane));  // the addresses below are formed here, not held through the strip
+            wave_fence();
+            v = sum_columns(lds, lane, W - x0);
+            wave_fence();  // the next part reuses the LDS
+        }
+        GlobalAS<double>* out = as_global(pdp->partials) + static_cast<uint64_t>(part) * 6u;
+        if (lane < 48u && (lane & 7u) == 0u) out[lane >> 3] = v;
     }
 }
 
@@ -1384,7 +1434,8 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const PairDes
         const bool active = level < plan->levels && (plan->mask[level] & (1u << c)) != 0u;
         double sum[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (active) {
-            const uint32_t begin = plan->item_begin[level][c], count = plan->item_count[level][c];
+            const uint32_t begin = plan->item_begin[level][c] << plan->part_shift;
+            const uint32_t count = plan->item_count[level][c] << plan->part_shift;
 #pragma unroll 4
             for (uint32_t it = lane; it < count; it += 64u) {
                 GlobalAS<const double>* p = partials + static_cast<uint64_t>(begin + it) * 6u;
@@ -1544,37 +1595,28 @@ hipError_t launch_prepare_t(MapForm map, bool general, const PairDesc* pairs, co
                : launch_prepare_m<Lay, false>(general, pairs, work, blocks, tiles, lut, src0, src1, persistent, stream);
 }
 
-template <typename Lay, typename TapsT, bool Ref, int Cols>
-hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t items,
+template <typename Lay, typename TapsT, bool Ref>
+hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t parts,
                           bool persistent, hipStream_t stream) {
-    const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref, Cols>, 64, blocks, persistent);
-    hipLaunchKernelGGL((scale_kernel<Lay, TapsT, Ref, Cols>), dim3(grid), dim3(64), 0, stream, pairs, work,
-                       blocks, items);
+    const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref>, 64, blocks, persistent);
+    hipLaunchKernelGGL((scale_kernel<Lay, TapsT, Ref>), dim3(grid), dim3(64), 0, stream, pairs, work, blocks, parts);
     return hipGetLastError();
 }
 
-template <typename Lay, bool Ref, int Cols>
+template <typename Lay, bool Ref>
 hipError_t launch_scale_m(uint32_t blur, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
-                          uint32_t items, bool persistent, hipStream_t stream) {
+                          uint32_t parts, bool persistent, hipStream_t stream) {
     return blur == kBlurRecursive
-               ? launch_scale_g<Lay, CosineTaps, Ref, Cols>(pairs, work, blocks, items, persistent, stream)
-               : launch_scale_g<Lay, SampledTaps, Ref, Cols>(pairs, work, blocks, items, persistent, stream);
-}
-
-template <typename Lay, int Cols>
-hipError_t launch_scale_c(uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
-                          uint32_t blocks, uint32_t items, bool persistent, hipStream_t stream) {
-    return map == kMapReference
-               ? launch_scale_m<Lay, true, Cols>(blur, pairs, work, blocks, items, persistent, stream)
-               : launch_scale_m<Lay, false, Cols>(blur, pairs, work, blocks, items, persistent, stream);
+               ? launch_scale_g<Lay, CosineTaps, Ref>(pairs, work, blocks, parts, persistent, stream)
+               : launch_scale_g<Lay, SampledTaps, Ref>(pairs, work, blocks, parts, persistent, stream);
 }
 
 template <typename Lay>
-hipError_t launch_scale_t(uint32_t strip_cols, uint32_t blur, MapForm map, const PairDesc* pairs,
-                          const WorkRef* work, uint32_t blocks, uint32_t items, bool persistent,
-                          hipStream_t stream) {
-    return strip_cols == 64 ? launch_scale_c<Lay, 1>(blur, map, pairs, work, blocks, items, persistent, stream)
-                            : launch_scale_c<Lay, 2>(blur, map, pairs, work, blocks, items, persistent, stream);
+hipError_t launch_scale_t(uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
+                          uint32_t parts, bool persistent, hipStream_t stream) {
+    return map == kMapReference
+               ? launch_scale_m<Lay, true>(blur, pairs, work, blocks, parts, persistent, stream)
+               : launch_scale_m<Lay, false>(blur, pairs, work, blocks, parts, persistent, stream);
 }
 
 }  // namespace
@@ -1625,18 +1667,16 @@ hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const Pa
     return hipErrorInvalidValue;
 }
 
-hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, uint32_t strip_cols,
-                       const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t items_per_pair,
-                       hipStream_t stream, bool persistent) {
+hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
+                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent) {
     if (blocks == 0) return hipSuccess;
-    if (blur > kBlurRecursive || map > kMapDifference || !ValidStripCols(strip_cols)) return hipErrorInvalidValue;
-    const uint32_t n = items_per_pair, sc = strip_cols;
+    if (blur > kBlurRecursive || map > kMapDifference) return hipErrorInvalidValue;
+    const uint32_t n = parts_per_pair;
     switch (format) {
-        case kPlaneF32: return launch_scale_t<LayoutF32>(sc, blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneF16: return launch_scale_t<LayoutF16>(sc, blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneBF16:
-            return launch_scale_t<LayoutBF16>(sc, blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneU16: return launch_scale_t<LayoutU16>(sc, blur, map, pairs, work, blocks, n, persistent, stream);
+        case kPlaneF32: return launch_scale_t<LayoutF32>(blur, map, pairs, work, blocks, n, persistent, stream);
+        case kPlaneF16: return launch_scale_t<LayoutF16>(blur, map, pairs, work, blocks, n, persistent, stream);
+        case kPlaneBF16: return launch_scale_t<LayoutBF16>(blur, map, pairs, work, blocks, n, persistent, stream);
+        case kPlaneU16: return launch_scale_t<LayoutU16>(blur, map, pairs, work, blocks, n, persistent, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -127,10 +127,12 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
     args.plan = FillPlan(config.width, config.height, format,
                          SinglePairStripRows(config.width, config.height, format, config.strip_rows,
                                              config.strip_cols),
-                         config.strip_cols);
+                         config.strip_cols,
+                         SinglePairRowParts(config.width, config.height, format, config.strip_rows, config.strip_cols));
     const Plan& p = args.plan;
+    const uint64_t parts = static_cast<uint64_t>(p.items) << p.part_shift;
     const uint64_t partials_at = Align256(kItemsAt + static_cast<uint64_t>(p.items) * sizeof(ScaleItem));
-    const uint64_t planes_at = Align256(partials_at + static_cast<uint64_t>(p.items) * 6 * sizeof(double));
+    const uint64_t planes_at = Align256(partials_at + parts * 6 * sizeof(double));
     const uint64_t need = planes_at + 2 * p.image_bytes;
     if (need > kNoAllocScratchBytes)
         Fail(VQM_INVALID_ARGUMENT,
@@ -161,7 +163,8 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
     const uint32_t tiles = p.prep_tiles_x * p.prep_tiles_y;
     Check(LaunchPrepare(format, map, false, dpair, nullptr, 2 * tiles, tiles, dlut, nullptr, nullptr, stream),
           "launch prepare");
-    Check(LaunchScale(format, config.blur, map, p.strip_w, dpair, nullptr, p.items, p.items, stream),
+    Check(LaunchScale(format, config.blur, map, dpair, nullptr, static_cast<uint32_t>(parts), static_cast<uint32_t>(parts),
+                      stream),
           "launch scale");
     Check(LaunchReduce(dpair, 1, stream), "launch reduce");
     return p.levels;

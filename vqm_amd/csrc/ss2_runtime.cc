@@ -148,8 +148,8 @@ DeviceContext& DeviceContext::Get() {
 }
 
 DevicePlan::DevicePlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
-                       uint32_t strip_cols)
-    : host(BuildPlan(width, height, format, strip_rows, strip_cols)),
+                       uint32_t strip_cols, uint32_t row_parts)
+    : host(BuildPlan(width, height, format, strip_rows, strip_cols, row_parts)),
       layout(LayoutWorkspace(host)),
       plan(sizeof(Plan)),
       items(std::max<uint64_t>(host.items.size(), 1) * sizeof(ScaleItem)) {
@@ -205,8 +205,9 @@ const DevicePlan& WorkspacePools::PlanFor(uint32_t width, uint32_t height) {
         const auto shape = shape_for_.find(std::make_pair(width, height));
         const bool set = shape != shape_for_.end();
         try {
-            slot = std::make_unique<DevicePlan>(width, height, format_, set ? shape->second.first : strip_rows_,
-                                                set ? shape->second.second : strip_cols_);
+            slot = set ? std::make_unique<DevicePlan>(width, height, format_, shape->second.rows, shape->second.cols,
+                                                      shape->second.row_parts)
+                       : std::make_unique<DevicePlan>(width, height, format_, strip_rows_, strip_cols_);
         } catch (...) {
             plans_.erase(std::make_pair(width, height));
             throw;
@@ -292,15 +293,14 @@ hipGraphExec_t Lane::CaptureGraph(PlaneFormat fmt, MapForm map, const float* lut
     const hipStream_t s = stream_.get();
     const GeometryPlan& g = plan.host;
     const PairDesc* dpairs = pairs_.as<PairDesc>();
-    const uint64_t prep = 2ull * g.prep_tiles * count, scale = static_cast<uint64_t>(g.plan.items) * count;
+    const uint64_t prep = 2ull * g.prep_tiles * count, scale = static_cast<uint64_t>(g.parts()) * count;
     Check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin graph capture");
     hipError_t e = hipMemcpyAsync(pairs_.get(), h_pairs_.get(), count * sizeof(PairDesc), hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
         e = LaunchPrepare(fmt, map, false, dpairs, nullptr, static_cast<uint32_t>(prep), g.prep_tiles, lut, nullptr,
                           nullptr, s, persistent);
     if (e == hipSuccess)
-        e = LaunchScale(fmt, blur, map, g.plan.strip_w, dpairs, nullptr, static_cast<uint32_t>(scale), g.plan.items, s,
-                        persistent);
+        e = LaunchScale(fmt, blur, map, dpairs, nullptr, static_cast<uint32_t>(scale), g.parts(), s, persistent);
     if (e == hipSuccess) e = LaunchReduce(dpairs, count, s);
     if (e == hipSuccess)
         e = hipMemcpyAsync(h_norms_.get(), norms_.get(), static_cast<uint64_t>(count) * kNorms * sizeof(double),
@@ -340,7 +340,7 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         general = general || e.general;
         uniform = uniform && e.plan == entries[0].plan;
         prep_work += 2ull * e.plan->host.prep_tiles;
-        scale_work += e.plan->host.plan.items;
+        scale_work += e.plan->host.parts();
         prep_at[i + 1] = prep_work;
         scale_at[i + 1] = scale_work;
     }
@@ -382,8 +382,6 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
     const WorkRef* wprep = nullptr;
     const WorkRef* wscale = nullptr;
     auto chunk_begin = [&](uint32_t c) { return static_cast<uint32_t>(uint64_t(c) * count / chunks); };
-    constexpr uint32_t kStripWidths[2] = {64, 128};
-    std::vector<uint64_t> scale_seg(2 * chunks + 1, 0);  // work-list runs by chunk and strip width
     if (!uniform) {
         if (h_work_prep_.bytes() < prep_work * sizeof(WorkRef)) {
             h_work_prep_ = PinnedBuffer(prep_work * sizeof(WorkRef));
@@ -400,20 +398,8 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
             const GeometryPlan& g = entries[i].plan->host;
             for (uint32_t image = 0; image < 2; ++image)
                 for (uint32_t k = 0; k < g.prep_tiles; ++k) wp[np++] = WorkRef{i, k | (image << 31)};
+            for (uint32_t k = 0; k < g.parts(); ++k) ws[ns++] = WorkRef{i, k};
         }
-        // Scale work, per chunk, in one run per strip width (each run is one
-        // launch of that width's kernel).
-        for (uint32_t c = 0; c < chunks; ++c) {
-            for (uint32_t g = 0; g < 2; ++g) {
-                scale_seg[2 * c + g] = ns;
-                for (uint32_t i = chunk_begin(c); i < chunk_begin(c + 1); ++i) {
-                    const Plan& p = entries[i].plan->host.plan;
-                    if (p.strip_w != kStripWidths[g]) continue;
-                    for (uint32_t k = 0; k < p.items; ++k) ws[ns++] = WorkRef{i, k};
-                }
-            }
-        }
-        scale_seg[2 * chunks] = ns;
         Check(hipMemcpyAsync(work_prep_.get(), wp, np * sizeof(WorkRef), hipMemcpyHostToDevice, s),
               "upload prepare work");
         Check(hipMemcpyAsync(work_scale_.get(), ws, ns * sizeof(WorkRef), hipMemcpyHostToDevice, s),
@@ -440,20 +426,10 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         const uint32_t i0 = chunk_begin(c), i1 = chunk_begin(c + 1);
         if (t != s) Check(hipStreamWaitEvent(t, Ev(4 * c + 1).get(), 0), "order scale after prepare");
         Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
-        if (uniform) {
-            const auto ns = static_cast<uint32_t>(scale_at[i1] - scale_at[i0]);
-            Check(LaunchScale(fmt, blur, map, g0.plan.strip_w, dpairs + i0, nullptr, ns, g0.plan.items, t,
-                              persistent),
-                  "launch scale");
-        } else {
-            for (uint32_t g = 0; g < 2; ++g) {
-                const auto ns = static_cast<uint32_t>(scale_seg[2 * c + g + 1] - scale_seg[2 * c + g]);
-                if (ns == 0) continue;
-                Check(LaunchScale(fmt, blur, map, kStripWidths[g], dpairs, wscale + scale_seg[2 * c + g], ns,
-                                  g0.plan.items, t, persistent),
-                      "launch scale");
-            }
-        }
+        const auto ns = static_cast<uint32_t>(scale_at[i1] - scale_at[i0]);
+        Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, uniform ? nullptr : wscale + scale_at[i0], ns,
+                          g0.parts(), t, persistent),
+              "launch scale");
         Check(hipEventRecord(Ev(4 * c + 3).get(), t), "hipEventRecord");
     }
     const uint32_t r = 4 * chunks;
@@ -529,7 +505,9 @@ Pipeline::Pipeline(const vqm_ss2_config& config)
       plan_(config.width, config.height, static_cast<PlaneFormat>(config.plane_format),
             SinglePairStripRows(config.width, config.height, static_cast<PlaneFormat>(config.plane_format),
                                 config.strip_rows, config.strip_cols),
-            config.strip_cols),
+            config.strip_cols,
+            SinglePairRowParts(config.width, config.height, static_cast<PlaneFormat>(config.plane_format),
+                               config.strip_rows, config.strip_cols)),
       ws_(plan_.layout),
       pair_(sizeof(PairDesc)),
       sources_(2 * sizeof(SourceDesc)),
@@ -616,7 +594,7 @@ void Pipeline::BuildGraph() {
     if (e == hipSuccess)
         e = LaunchPrepare(fmt, map_, false, pd, nullptr, 2 * g.prep_tiles, g.prep_tiles, ctx_.lut, nullptr, nullptr, s);
     if (e == hipSuccess)
-        e = LaunchScale(fmt, config_.blur, map_, g.plan.strip_w, pd, nullptr, g.plan.items, g.plan.items, s);
+        e = LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s);
     if (e == hipSuccess) e = LaunchReduce(pd, 1, s);
     if (e == hipSuccess)
         e = hipMemcpyAsync(host_norms_.get(), ws_.norms, kNorms * sizeof(double), hipMemcpyDeviceToHost, s);
@@ -709,7 +687,7 @@ uint64_t Pipeline::Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_o
                             s),
               "launch prepare");
     Check(hipEventRecord(ev_[1].get(), s), "hipEventRecord");
-    Check(LaunchScale(fmt, config_.blur, map_, g.plan.strip_w, pd, nullptr, g.plan.items, g.plan.items, s),
+    Check(LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s),
           "launch scale");
     Check(hipEventRecord(ev_[2].get(), s), "hipEventRecord");
     Check(LaunchReduce(pd, 1, s), "launch reduce");
@@ -917,14 +895,14 @@ const vqm_ss2_batch_config& ValidatedBatch(const vqm_ss2_batch_config& config) {
 }
 }  // namespace
 
-// A batch's default strip height for a geometry, chosen when the geometry
-// is first submitted with `pairs` pairs of it (DefaultStripRows). Measured on
-// 300 1080p pairs, 192 rows run the scale launch 2.5% faster than 128 (as
-// fast as 256, with less padding); one 1080p pair takes 6.5k pairs/s at 64
-// rows and 3.6k at 192.
-uint32_t Batch::DefaultStripRows(uint32_t width, uint32_t height, uint32_t pairs) const {
-    return ss2::DefaultStripRows(width, height, static_cast<PlaneFormat>(config_.plane_format), config_.strip_cols,
-                                 pairs, static_cast<uint32_t>(std::max(ctx_.cus, 1)));
+// A batch's default strip shape for a geometry, chosen when the geometry is
+// first submitted with `pairs` pairs of it (DefaultStripRows, RowParts).
+void Batch::SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs) {
+    const auto format = static_cast<PlaneFormat>(config_.plane_format);
+    const auto cus = static_cast<uint32_t>(std::max(ctx_.cus, 1));
+    const uint32_t rows = DefaultStripRows(width, height, format, config_.strip_cols, pairs, cus);
+    pools_.SetStripShape(width, height, rows, config_.strip_cols,
+                         RowParts(width, height, format, rows, config_.strip_cols, pairs, cus));
 }
 
 Batch::Batch(const vqm_ss2_batch_config& config)
@@ -977,7 +955,7 @@ uint64_t Batch::Submit(const vqm_ss2_device_pair* pairs, uint32_t count) {
     for (const auto& [geometry, n] : per_geometry) {
         const auto [w, h] = geometry;
         if (config_.strip_rows == 0 && !pools_.HasPlan(w, h) && !pools_.HasShape(w, h))
-            pools_.SetStripShape(w, h, DefaultStripRows(w, h, n), config_.strip_cols);
+            SetDefaultShape(w, h, n);
         pools_.PlanFor(w, h);
     }
     std::vector<Taken> taken;

@@ -118,7 +118,8 @@ struct DevicePlan {
     WorkspaceLayout layout;
     DeviceBuffer plan;   // one Plan
     DeviceBuffer items;  // ScaleItem[items]
-    DevicePlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols);
+    DevicePlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
+               uint32_t row_parts = 1);
 };
 
 // One pair's device workspace: planes (zero borders), partials, norms and,
@@ -170,9 +171,10 @@ public:
     bool HasPlan(uint32_t width, uint32_t height) const {
         return plans_.count(std::make_pair(width, height)) != 0;
     }
-    // The strip height and width of a geometry whose plan does not exist yet.
-    void SetStripShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint32_t strip_cols) {
-        shape_for_[std::make_pair(width, height)] = std::make_pair(strip_rows, strip_cols);
+    // The strip shape of a geometry whose plan does not exist yet.
+    void SetStripShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint32_t strip_cols,
+                       uint32_t row_parts = 1) {
+        shape_for_[std::make_pair(width, height)] = StripShape{strip_rows, strip_cols, row_parts};
     }
     bool HasShape(uint32_t width, uint32_t height) const {
         return shape_for_.count(std::make_pair(width, height)) != 0;
@@ -195,6 +197,9 @@ private:
             return std::tie(width, height, inputs) < std::tie(o.width, o.height, o.inputs);
         }
     };
+    struct StripShape {
+        uint32_t rows, cols, row_parts;
+    };
     struct Pool {
         std::vector<std::unique_ptr<Workspace>> idle;
         uint64_t each = 0;
@@ -205,7 +210,7 @@ private:
     uint64_t budget_;
     std::unique_ptr<Arena> arena_;
     std::map<std::pair<uint32_t, uint32_t>, std::unique_ptr<DevicePlan>> plans_;
-    std::map<std::pair<uint32_t, uint32_t>, std::pair<uint32_t, uint32_t>> shape_for_;
+    std::map<std::pair<uint32_t, uint32_t>, StripShape> shape_for_;
     std::map<Key, Pool> pools_;
     uint64_t bytes_ = 0, peak_ = 0;
 };
@@ -402,7 +407,7 @@ public:
     // Fixes the strip shape of a geometry not used yet (a shape tuned
     // earlier, or by another process).
     void SetShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint32_t strip_cols);
-    uint32_t DefaultStripRows(uint32_t width, uint32_t height, uint32_t pairs) const;
+    void SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs);
 
 private:
     struct Taken {

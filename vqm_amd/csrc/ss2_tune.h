@@ -1,8 +1,6 @@
 // Launch-shape autotuner: picks the scale strip height and width and the
 // batch chunk count for a geometry, plane format and batch size by timing
-// every candidate on the device. The strip width also picks the scale
-// kernel's occupancy (one output column per lane holds half the register
-// ring of two). No shape changes a pixel's arithmetic or an FP32 block sum;
+// every candidate on the device. No shape changes a pixel's arithmetic or an FP32 block sum;
 // only the order of the FP64 strip partials follows the strips, so the
 // choice is free to follow the measurement. Choices are cached per (width,
 // height, format, map form, batch-size class) for the process.
