@@ -39,8 +39,9 @@ inline constexpr uint32_t kSumBlockRows = 8;
 inline constexpr int kPadTop = kRadius;
 inline constexpr int kPadLeft = 8;
 
-// Prepare kernel: a 256-thread block converts a 64 x 32 base-pixel tile and
-// every level of its sub-pyramid (64 x 32 halves down to 2 x 1 at level 5).
+// Prepare kernel: tiles of 64 x 32 base pixels, with every level of their
+// sub-pyramid that stores a channel (levels 0 to 4; 64 x 32 halves down to
+// 4 x 2); a wave takes the upper or lower half of one.
 inline constexpr int kPrepTileW = 64;
 inline constexpr int kPrepTileH = 32;
 

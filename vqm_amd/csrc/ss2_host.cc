@@ -262,6 +262,9 @@ Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t stri
             cursor = Align(cursor + CheckedMul(CheckedMul(p.pitch[l], p.rows[l]), ElementBytes(format)), 256);
         }
     }
+    // The prepare kernel stops at level 4: six scales' pruning leaves level 5
+    // no stored channel.
+    if (p.mask[kMaxScales - 1] != 0u) Fail(VQM_RUNTIME_ERROR, "level 5 stores a channel");
     p.image_bytes = cursor;
     // Scale work: per level and active channel, bands of strip_rows rows by
     // strip_cols-column strips, row-major so that consecutive items are
