@@ -12,7 +12,8 @@
 //            padding of the 13-tap blur (scale.comp:107-124), so the scale
 //            kernel loads whole rows without bounds checks.
 //   partials items x 6 doubles: one FP64 partial per scale work item.
-//   norms    108 doubles: the finished norms of the pair.
+// The pair's 108 norms go to pinned host memory, or to a device buffer of the
+// caller's.
 #pragma once
 
 #include <cstdint>

@@ -362,8 +362,7 @@ WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan) {
     WorkspaceLayout l;
     l.planes = Align(2 * plan.plane_bytes_per_image, 256);
     l.partials = Align((static_cast<uint64_t>(std::max(plan.plan.items, 1u)) << plan.plan.part_shift) * 6 * sizeof(double), 256);
-    l.norms = Align(kNorms * sizeof(double), 256);
-    l.total = l.planes + l.partials + l.norms;
+    l.total = l.planes + l.partials;
     return l;
 }
 

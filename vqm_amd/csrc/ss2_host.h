@@ -122,10 +122,10 @@ uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t 
 uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                             uint32_t strip_cols);
 
-// Bytes of one pair's workspace: planes of both images, partials, norms,
-// each rounded to 256 bytes.
+// Bytes of one pair's workspace: planes of both images and partials, each
+// rounded to 256 bytes.
 struct WorkspaceLayout {
-    uint64_t planes = 0, partials = 0, norms = 0, total = 0;
+    uint64_t planes = 0, partials = 0, total = 0;
 };
 WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan);
 

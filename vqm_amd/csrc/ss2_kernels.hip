@@ -31,6 +31,7 @@
 // loads; images and planes through global-address-space pointers.
 
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include <algorithm>
 #include <cstdint>
@@ -1715,56 +1716,70 @@ uint32_t GridOf(K kernel, int block_threads, uint32_t blocks, bool persistent) {
     return resident == 0 ? blocks : std::min(blocks, resident);
 }
 
+// Launches `kernel`, with `done` (null: none) set by its own dispatch.
+template <typename... Params, typename... Args>
+hipError_t Dispatch(void (*kernel)(Params...), uint32_t grid, uint32_t threads, hipStream_t stream, hipEvent_t done,
+                    Args... args) {
+    if (done != nullptr)
+        hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, nullptr, done, 0,
+                              static_cast<Params>(args)...);
+    else
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, static_cast<Params>(args)...);
+    return hipGetLastError();
+}
+
+// A launch of no work: `done` still follows what is queued.
+hipError_t Nothing(hipStream_t stream, hipEvent_t done) {
+    return done != nullptr ? hipEventRecord(done, stream) : hipSuccess;
+}
+
 template <typename Lay, bool General, bool Ref>
 hipError_t launch_prepare_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t tiles,
                             const float* lut, const uint8_t* src0, const uint8_t* src1, bool persistent,
-                            hipStream_t stream) {
+                            hipStream_t stream, hipEvent_t done) {
     constexpr uint32_t kThreads = 64 * kPrepWaves<General>, kBlocksPerTile = kPrepTileH / kWaveRows / kPrepWaves<General>;
     const uint32_t grid = GridOf(&prepare_kernel<Lay, General, Ref>, kThreads, blocks * kBlocksPerTile, persistent);
-    hipLaunchKernelGGL((prepare_kernel<Lay, General, Ref>), dim3(grid), dim3(kThreads), 0, stream, pairs, work,
-                       blocks, tiles, lut, src0, src1);
-    return hipGetLastError();
+    return Dispatch(&prepare_kernel<Lay, General, Ref>, grid, kThreads, stream, done, pairs, work, blocks, tiles, lut,
+                    src0, src1);
 }
 
 template <typename Lay, bool Ref>
 hipError_t launch_prepare_m(bool general, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
                             uint32_t tiles, const float* lut, const uint8_t* src0, const uint8_t* src1,
-                            bool persistent, hipStream_t stream) {
-    return general ? launch_prepare_g<Lay, true, Ref>(pairs, work, blocks, tiles, lut, src0, src1, persistent, stream)
-                   : launch_prepare_g<Lay, false, Ref>(pairs, work, blocks, tiles, lut, src0, src1, persistent, stream);
+                            bool persistent, hipStream_t stream, hipEvent_t done) {
+    const auto launch = general ? &launch_prepare_g<Lay, true, Ref> : &launch_prepare_g<Lay, false, Ref>;
+    return launch(pairs, work, blocks, tiles, lut, src0, src1, persistent, stream, done);
 }
 
 template <typename Lay>
 hipError_t launch_prepare_t(MapForm map, bool general, const PairDesc* pairs, const WorkRef* work,
                             uint32_t blocks, uint32_t tiles, const float* lut, const uint8_t* src0,
-                            const uint8_t* src1, bool persistent, hipStream_t stream) {
-    return map == kMapReference
-               ? launch_prepare_m<Lay, true>(general, pairs, work, blocks, tiles, lut, src0, src1, persistent, stream)
-               : launch_prepare_m<Lay, false>(general, pairs, work, blocks, tiles, lut, src0, src1, persistent, stream);
+                            const uint8_t* src1, bool persistent, hipStream_t stream, hipEvent_t done) {
+    const auto launch = map == kMapReference ? &launch_prepare_m<Lay, true> : &launch_prepare_m<Lay, false>;
+    return launch(general, pairs, work, blocks, tiles, lut, src0, src1, persistent, stream, done);
 }
 
 template <typename Lay, typename TapsT, bool Ref>
 hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t parts,
-                          bool persistent, hipStream_t stream) {
+                          bool persistent, hipStream_t stream, hipEvent_t done) {
     const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref>, 64, blocks, persistent);
-    hipLaunchKernelGGL((scale_kernel<Lay, TapsT, Ref>), dim3(grid), dim3(64), 0, stream, pairs, work, blocks, parts);
-    return hipGetLastError();
+    return Dispatch(&scale_kernel<Lay, TapsT, Ref>, grid, 64, stream, done, pairs, work, blocks, parts);
 }
 
 template <typename Lay, bool Ref>
 hipError_t launch_scale_m(uint32_t blur, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
-                          uint32_t parts, bool persistent, hipStream_t stream) {
+                          uint32_t parts, bool persistent, hipStream_t stream, hipEvent_t done) {
     return blur == kBlurRecursive
-               ? launch_scale_g<Lay, CosineTaps, Ref>(pairs, work, blocks, parts, persistent, stream)
-               : launch_scale_g<Lay, SampledTaps, Ref>(pairs, work, blocks, parts, persistent, stream);
+               ? launch_scale_g<Lay, CosineTaps, Ref>(pairs, work, blocks, parts, persistent, stream, done)
+               : launch_scale_g<Lay, SampledTaps, Ref>(pairs, work, blocks, parts, persistent, stream, done);
 }
 
 template <typename Lay>
 hipError_t launch_scale_t(uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
-                          uint32_t parts, bool persistent, hipStream_t stream) {
+                          uint32_t parts, bool persistent, hipStream_t stream, hipEvent_t done) {
     return map == kMapReference
-               ? launch_scale_m<Lay, true>(blur, pairs, work, blocks, parts, persistent, stream)
-               : launch_scale_m<Lay, false>(blur, pairs, work, blocks, parts, persistent, stream);
+               ? launch_scale_m<Lay, true>(blur, pairs, work, blocks, parts, persistent, stream, done)
+               : launch_scale_m<Lay, false>(blur, pairs, work, blocks, parts, persistent, stream, done);
 }
 
 }  // namespace
@@ -1794,45 +1809,46 @@ hipError_t LaunchCbrtCheck(uint32_t first, uint32_t end, CbrtCheck* out, hipStre
 
 hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const PairDesc* pairs,
                          const WorkRef* work, uint32_t blocks, uint32_t tiles_per_image, const float* lut,
-                         const uint8_t* src0, const uint8_t* src1, hipStream_t stream, bool persistent) {
-    if (blocks == 0) return hipSuccess;
+                         const uint8_t* src0, const uint8_t* src1, hipStream_t stream, bool persistent,
+                         hipEvent_t done) {
+    if (blocks == 0) return Nothing(stream, done);
     if (map > kMapDifference) return hipErrorInvalidValue;
     const uint32_t t = tiles_per_image;
     switch (format) {
         case kPlaneF32:
             return launch_prepare_t<LayoutF32>(map, general, pairs, work, blocks, t, lut, src0, src1, persistent,
-                                               stream);
+                                              stream, done);
         case kPlaneF16:
             return launch_prepare_t<LayoutF16>(map, general, pairs, work, blocks, t, lut, src0, src1, persistent,
-                                               stream);
+                                              stream, done);
         case kPlaneBF16:
             return launch_prepare_t<LayoutBF16>(map, general, pairs, work, blocks, t, lut, src0, src1, persistent,
-                                                stream);
+                                               stream, done);
         case kPlaneU16:
             return launch_prepare_t<LayoutU16>(map, general, pairs, work, blocks, t, lut, src0, src1, persistent,
-                                               stream);
+                                              stream, done);
     }
     return hipErrorInvalidValue;
 }
 
 hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
-                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent) {
-    if (blocks == 0) return hipSuccess;
+                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent,
+                       hipEvent_t done) {
+    if (blocks == 0) return Nothing(stream, done);
     if (blur > kBlurRecursive || map > kMapDifference) return hipErrorInvalidValue;
     const uint32_t n = parts_per_pair;
     switch (format) {
-        case kPlaneF32: return launch_scale_t<LayoutF32>(blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneF16: return launch_scale_t<LayoutF16>(blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneBF16: return launch_scale_t<LayoutBF16>(blur, map, pairs, work, blocks, n, persistent, stream);
-        case kPlaneU16: return launch_scale_t<LayoutU16>(blur, map, pairs, work, blocks, n, persistent, stream);
+        case kPlaneF32: return launch_scale_t<LayoutF32>(blur, map, pairs, work, blocks, n, persistent, stream, done);
+        case kPlaneF16: return launch_scale_t<LayoutF16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
+        case kPlaneBF16: return launch_scale_t<LayoutBF16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
+        case kPlaneU16: return launch_scale_t<LayoutU16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
     }
     return hipErrorInvalidValue;
 }
 
-hipError_t LaunchReduce(const PairDesc* pairs, uint32_t pairs_count, hipStream_t stream) {
-    if (pairs_count == 0) return hipSuccess;
-    hipLaunchKernelGGL(reduce_kernel, dim3(pairs_count), dim3(64 * kReduceWaves), 0, stream, pairs);
-    return hipGetLastError();
+hipError_t LaunchReduce(const PairDesc* pairs, uint32_t pairs_count, hipStream_t stream, hipEvent_t done) {
+    if (pairs_count == 0) return Nothing(stream, done);
+    return Dispatch(&reduce_kernel, pairs_count, 64 * kReduceWaves, stream, done, pairs);
 }
 
 }  // namespace vqm::ss2

@@ -83,9 +83,9 @@ DeviceBuffer& DeviceBuffer::operator=(DeviceBuffer&& o) noexcept {
     return *this;
 }
 
-PinnedBuffer::PinnedBuffer(uint64_t bytes) : bytes_(bytes) {
+PinnedBuffer::PinnedBuffer(uint64_t bytes, bool kernel_writes) : bytes_(bytes) {
     if (bytes == 0) return;
-    if (hipHostMalloc(&ptr_, bytes, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&ptr_, bytes, kernel_writes ? hipHostMallocCoherent : hipHostMallocDefault) != hipSuccess) {
         ptr_ = nullptr;
         (void)hipGetLastError();
         Fail(VQM_RUNTIME_ERROR, "hip: pinned host allocation of " + std::to_string(bytes) + " bytes failed");
@@ -185,7 +185,6 @@ Workspace::Workspace(const WorkspaceLayout& layout, uint64_t input_image_bytes, 
     Check(hipStreamSynchronize(nullptr), "clear workspace");
     planes = base;
     partials = reinterpret_cast<double*>(base + layout.planes);
-    norms = reinterpret_cast<double*>(base + layout.planes + layout.partials);
     if (input_image_bytes > 0) inputs = base + layout.total;
 }
 
@@ -272,11 +271,10 @@ void WorkspacePools::Return(uint32_t width, uint32_t height, bool inputs, std::u
 Lane::Lane(uint32_t max_pairs, uint32_t graphs)
     : max_pairs_(max_pairs),
       pairs_(max_pairs * sizeof(PairDesc)),
-      norms_(static_cast<uint64_t>(max_pairs) * kNorms * sizeof(double)),
       h_pairs_(max_pairs * sizeof(PairDesc)),
-      h_norms_(static_cast<uint64_t>(max_pairs) * kNorms * sizeof(double)),
+      h_norms_(static_cast<uint64_t>(max_pairs) * kNorms * sizeof(double), true),
       graphs_(graphs) {
-    for (uint32_t i = 0; i < 4 * kMaxChunks + 3; ++i) ev_.push_back(std::make_unique<Event>());
+    for (uint32_t i = 0; i < 4 * kMaxChunks + 1; ++i) ev_.push_back(std::make_unique<Event>());
 }
 
 Lane::~Lane() {
@@ -287,7 +285,7 @@ Lane::~Lane() {
 // Captures one launch shape on the lane's first stream: the upload of the
 // pinned pair descriptors (rewritten before every replay: workspaces and
 // inputs change), the prepare, scale and reduce kernels over `count` pairs
-// of `plan`, and the read-back of their norms.
+// of `plan`, which write their norms to pinned host memory.
 hipGraphExec_t Lane::CaptureGraph(PlaneFormat fmt, MapForm map, const float* lut, const DevicePlan& plan,
                                   uint32_t count, uint32_t blur, bool persistent) {
     const hipStream_t s = stream_.get();
@@ -302,9 +300,6 @@ hipGraphExec_t Lane::CaptureGraph(PlaneFormat fmt, MapForm map, const float* lut
     if (e == hipSuccess)
         e = LaunchScale(fmt, blur, map, dpairs, nullptr, static_cast<uint32_t>(scale), g.parts(), s, persistent);
     if (e == hipSuccess) e = LaunchReduce(dpairs, count, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(h_norms_.get(), norms_.get(), static_cast<uint64_t>(count) * kNorms * sizeof(double),
-                           hipMemcpyDeviceToHost, s);
     hipGraph_t graph = nullptr;
     const hipError_t end = hipStreamEndCapture(s, &graph);
     Check(e, "capture a batch launch");
@@ -332,7 +327,7 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
             pd.src[k] = e.host[k] ? e.ws->inputs + k * ((e.image_bytes + 255) / 256 * 256) : e.src[k];
         pd.planes = e.ws->planes;
         pd.partials = e.ws->partials;
-        pd.norms = norms_.as<double>() + static_cast<uint64_t>(i) * kNorms;
+        pd.norms = h_norms_.as<double>() + static_cast<uint64_t>(i) * kNorms;
         pd.plan = e.plan->plan.as<Plan>();
         pd.items = e.plan->items.as<ScaleItem>();
         pd.source[0] = e.source[0];
@@ -418,28 +413,21 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         const WorkRef* wp = uniform ? nullptr : wprep + prep_at[i0];
         const auto np = static_cast<uint32_t>(prep_at[i1] - prep_at[i0]);
         Check(hipEventRecord(Ev(4 * c).get(), s), "hipEventRecord");
-        Check(LaunchPrepare(fmt, map, general, base, wp, np, g0.prep_tiles, lut, nullptr, nullptr, s, persistent),
+        Check(LaunchPrepare(fmt, map, general, base, wp, np, g0.prep_tiles, lut, nullptr, nullptr, s, persistent,
+                            chunks == 1 ? Ev(1).get() : nullptr),
               "launch prepare");
-        Check(hipEventRecord(Ev(4 * c + 1).get(), s), "hipEventRecord");
+        if (chunks > 1) Check(hipEventRecord(Ev(4 * c + 1).get(), s), "hipEventRecord");
     }
     for (uint32_t c = 0; c < chunks; ++c) {
         const uint32_t i0 = chunk_begin(c), i1 = chunk_begin(c + 1);
         if (t != s) Check(hipStreamWaitEvent(t, Ev(4 * c + 1).get(), 0), "order scale after prepare");
-        Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
         const auto ns = static_cast<uint32_t>(scale_at[i1] - scale_at[i0]);
+        if (t != s) Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
         Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, uniform ? nullptr : wscale + scale_at[i0], ns,
-                          g0.parts(), t, persistent),
+                          g0.parts(), t, persistent, Ev(4 * c + 3).get()),
               "launch scale");
-        Check(hipEventRecord(Ev(4 * c + 3).get(), t), "hipEventRecord");
     }
-    const uint32_t r = 4 * chunks;
-    Check(hipEventRecord(Ev(r).get(), t), "hipEventRecord");
-    Check(LaunchReduce(dpairs, count, t), "launch reduce");
-    Check(hipEventRecord(Ev(r + 1).get(), t), "hipEventRecord");
-    Check(hipMemcpyAsync(h_norms_.get(), norms_.get(), static_cast<uint64_t>(count) * kNorms * sizeof(double),
-                         hipMemcpyDeviceToHost, t),
-          "read back norms");
-    Check(hipEventRecord(Ev(r + 2).get(), t), "hipEventRecord");
+    Check(LaunchReduce(dpairs, count, t, Ev(DoneEvent()).get()), "launch reduce");
     pending_ = true;
 }
 
@@ -470,9 +458,9 @@ std::array<float, 3> Lane::StageTimes() const {
     }
     for (uint32_t c = 0; c < chunks_; ++c) {
         t[0] += Elapsed(Ev(4 * c), Ev(4 * c + 1));
-        t[1] += Elapsed(Ev(4 * c + 2), Ev(4 * c + 3));
+        t[1] += Elapsed(Ev(chunks_ == 1 ? 1 : 4 * c + 2), Ev(4 * c + 3));
     }
-    t[2] = Elapsed(Ev(4 * chunks_), Ev(4 * chunks_ + 1));
+    t[2] = Elapsed(Ev(4 * chunks_ - 1), Ev(DoneEvent()));
     return t;
 }
 
@@ -520,7 +508,8 @@ Pipeline::Pipeline(const vqm_ss2_config& config)
     PairDesc pd{};
     pd.planes = ws_.planes;
     pd.partials = ws_.partials;
-    pd.norms = ws_.norms;
+    host_norms_ = PinnedBuffer(kNorms * sizeof(double), true);
+    pd.norms = host_norms_.as<double>();
     pd.plan = plan_.plan.as<Plan>();
     pd.items = plan_.items.as<ScaleItem>();
     pd.source[0] = sources_.as<SourceDesc>();
@@ -535,7 +524,6 @@ Pipeline::Pipeline(const vqm_ss2_config& config)
     slots_.resize(config.resident_images);
     for (Slot& s : slots_) s.data = DeviceBuffer(image_bytes_);
     if (config.streaming_inputs) EnsureStreaming(image_bytes_);
-    host_norms_ = PinnedBuffer(kNorms * sizeof(double));
     if (config.input_bytes > 0) input_pool_ = DeviceBuffer(config.input_bytes);
     if (config.resident_images > 0) {
         // The prepare work of the distorted image alone, for pairs whose
@@ -550,7 +538,7 @@ Pipeline::Pipeline(const vqm_ss2_config& config)
 }
 
 Pipeline::~Pipeline() {
-    if (in_flight_ != 0) (void)hipEventSynchronize(ev_[4].get());
+    if (in_flight_ != 0) (void)hipEventSynchronize(ev_[3].get());
     if (graph_) (void)hipGraphExecDestroy(graph_);
 }
 
@@ -580,10 +568,11 @@ void Pipeline::SetSources(const vqm_image_format& a, const vqm_image_format& b, 
 }
 
 // Captures, on the pipeline's stream, the upload of the pinned pair
-// descriptor (its input pointers change per pair), the three kernels (the
-// prepare kernel reads its inputs through the descriptor) and the norm
-// read-back. The graph holds no memset node: the plane borders are cleared
-// once, when the workspace is created. Graphs cover 8-bit sRGB RGB pairs.
+// descriptor (its input pointers change per pair) and the three kernels (the
+// prepare kernel reads its inputs through the descriptor; the reduce writes
+// the norms to pinned host memory). The graph holds no memset node: the plane
+// borders are cleared once, when the workspace is created. Graphs cover 8-bit
+// sRGB RGB pairs.
 void Pipeline::BuildGraph() {
     const hipStream_t s = stream_.get();
     const PairDesc* pd = pair_.as<PairDesc>();
@@ -596,8 +585,6 @@ void Pipeline::BuildGraph() {
     if (e == hipSuccess)
         e = LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s);
     if (e == hipSuccess) e = LaunchReduce(pd, 1, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(host_norms_.get(), ws_.norms, kNorms * sizeof(double), hipMemcpyDeviceToHost, s);
     hipGraph_t graph = nullptr;
     const hipError_t end = hipStreamEndCapture(s, &graph);
     Check(e, "capture the pair's launches");
@@ -666,7 +653,7 @@ uint64_t Pipeline::Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_o
         hp->src[1] = src1;
         Check(hipEventRecord(ev_[0].get(), s), "hipEventRecord");
         Check(hipGraphLaunch(graph_, s), "launch the pair's graph");
-        Check(hipEventRecord(ev_[4].get(), s), "hipEventRecord");
+        Check(hipEventRecord(ev_[3].get(), s), "hipEventRecord");
         graph_launched_ = true;
         in_flight_ = NextId();
         return in_flight_;
@@ -678,24 +665,15 @@ uint64_t Pipeline::Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_o
         sources_pending_ = false;
     }
     Check(hipEventRecord(ev_[0].get(), s), "hipEventRecord");
-    if (reuse_original)
-        Check(LaunchPrepare(fmt, map_, general_, pd, distorted_work_.as<WorkRef>(), g.prep_tiles, g.prep_tiles,
-                            ctx_.lut, src0, src1, s),
-              "launch prepare");
-    else
-        Check(LaunchPrepare(fmt, map_, general_, pd, nullptr, 2 * g.prep_tiles, g.prep_tiles, ctx_.lut, src0, src1,
-                            s),
-              "launch prepare");
-    Check(hipEventRecord(ev_[1].get(), s), "hipEventRecord");
-    Check(LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s),
+    Check(reuse_original
+              ? LaunchPrepare(fmt, map_, general_, pd, distorted_work_.as<WorkRef>(), g.prep_tiles, g.prep_tiles,
+                              ctx_.lut, src0, src1, s, false, ev_[1].get())
+              : LaunchPrepare(fmt, map_, general_, pd, nullptr, 2 * g.prep_tiles, g.prep_tiles, ctx_.lut, src0, src1,
+                              s, false, ev_[1].get()),
+          "launch prepare");
+    Check(LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s, false, ev_[2].get()),
           "launch scale");
-    Check(hipEventRecord(ev_[2].get(), s), "hipEventRecord");
-    Check(LaunchReduce(pd, 1, s), "launch reduce");
-    Check(hipEventRecord(ev_[3].get(), s), "hipEventRecord");
-    Check(hipMemcpyAsync(host_norms_.get(), ws_.norms, kNorms * sizeof(double),
-                         hipMemcpyDeviceToHost, s),
-          "read back norms");
-    Check(hipEventRecord(ev_[4].get(), s), "hipEventRecord");
+    Check(LaunchReduce(pd, 1, s, ev_[3].get()), "launch reduce");
     in_flight_ = NextId();
     return in_flight_;
 }
@@ -851,7 +829,7 @@ uint64_t Pipeline::SubmitBuffers(uint64_t a, uint64_t b, float background) {
 uint32_t Pipeline::Finish(uint64_t token, double* norms) {
     if (token == 0 || token != in_flight_)
         Fail(VQM_INVALID_ARGUMENT, "unknown or already finished submission token");
-    const hipError_t waited = hipEventSynchronize(ev_[4].get());
+    const hipError_t waited = hipEventSynchronize(ev_[3].get());
     in_flight_ = 0;
     if (waited != hipSuccess) {
         // The pair's work may still touch the staging and the workspace:
@@ -860,7 +838,7 @@ uint32_t Pipeline::Finish(uint64_t token, double* norms) {
         Check(waited, "wait for pair");
     }
     if (graph_launched_)
-        stage_ms_ = {Elapsed(ev_[0], ev_[4]), 0.0f, 0.0f};
+        stage_ms_ = {Elapsed(ev_[0], ev_[3]), 0.0f, 0.0f};
     else
         stage_ms_ = {Elapsed(ev_[0], ev_[1]), Elapsed(ev_[1], ev_[2]), Elapsed(ev_[2], ev_[3])};
     std::memcpy(norms, host_norms_.get(), kNorms * sizeof(double));

@@ -48,7 +48,8 @@ private:
 class PinnedBuffer {
 public:
     PinnedBuffer() = default;
-    explicit PinnedBuffer(uint64_t bytes);
+    // kernel_writes: fine-grained memory, for kernels to write results to.
+    explicit PinnedBuffer(uint64_t bytes, bool kernel_writes = false);
     ~PinnedBuffer();
     PinnedBuffer(PinnedBuffer&& o) noexcept : ptr_(std::exchange(o.ptr_, nullptr)), bytes_(std::exchange(o.bytes_, 0)) {}
     PinnedBuffer& operator=(PinnedBuffer&& o) noexcept;
@@ -122,7 +123,7 @@ struct DevicePlan {
                uint32_t row_parts = 1);
 };
 
-// One pair's device workspace: planes (zero borders), partials, norms and,
+// One pair's device workspace: planes (zero borders), partials and,
 // for pairs whose inputs arrive from the host, room for both input images.
 // It owns its memory, or uses `bytes` at `memory` carved from an arena.
 struct Workspace {
@@ -131,7 +132,6 @@ struct Workspace {
     uint64_t bytes = 0;
     void* planes = nullptr;
     double* partials = nullptr;
-    double* norms = nullptr;
     uint8_t* inputs = nullptr;  // 2 * input_image_bytes, or null
     Workspace(const WorkspaceLayout& layout, uint64_t input_image_bytes = 0, void* memory = nullptr);
     // Bytes a workspace of this layout needs.
@@ -244,8 +244,8 @@ public:
     // HIP graphs (see Launch); 2 only those of up to kAutoGraphPairs pairs.
     explicit Lane(uint32_t max_pairs, uint32_t graphs = 0);
     ~Lane();
-    // Queues the uploads, the prepare, scale and reduce launches and the norm
-    // read-back, then returns. With chunks > 1 the pairs are split into that
+    // Queues the uploads and the prepare, scale and reduce launches (the last
+    // writes the norms to pinned host memory), then returns. With chunks > 1 the pairs are split into that
     // many runs of consecutive pairs: the prepare launches of the runs follow
     // one another on the lane's first stream, and each run's scale launch
     // follows on a second stream as soon as its prepare is done, so the
@@ -256,8 +256,8 @@ public:
     // geometry, one run, 8-bit sRGB device inputs is replayed from a HIP
     // graph captured the first time its shape (plan, pair count, format,
     // map form, blur, persistent) is seen: the descriptor upload from the
-    // pinned descriptors written for this launch, the three kernels and the
-    // norm read-back, as one submission. It holds no memset node.
+    // pinned descriptors written for this launch and the three kernels, as
+    // one submission. It holds no memset node.
     void Launch(PlaneFormat format, MapForm map, const float* lut, const LaunchEntry* entries,
                 uint32_t count, uint32_t chunks = 1, uint32_t blur = kBlurSampled,
                 bool persistent = false);
@@ -279,11 +279,11 @@ public:
 
 private:
     uint32_t max_pairs_;
-    DeviceBuffer pairs_, work_prep_, work_scale_, norms_;
+    DeviceBuffer pairs_, work_prep_, work_scale_;
     PinnedBuffer h_pairs_, h_work_prep_, h_work_scale_, h_norms_;
     Stream stream_, scale_stream_;
-    // Per chunk: prepare start/end, scale start/end; then reduce start/end
-    // and the end of the read-back.
+    // Per chunk: prepare start/end, scale start (on its own stream; unused
+    // with one chunk)/end; then reduce end.
     std::vector<std::unique_ptr<Event>> ev_;
     uint32_t chunks_ = 1;
     bool pending_ = false;
@@ -303,7 +303,7 @@ private:
                                 uint32_t count, uint32_t blur, bool persistent);
     Event& Ev(uint32_t i) { return *ev_[i]; }
     const Event& Ev(uint32_t i) const { return *ev_[i]; }
-    uint32_t DoneEvent() const { return 4 * chunks_ + 2; }
+    uint32_t DoneEvent() const { return 4 * chunks_; }
 };
 
 class Pipeline {
@@ -379,7 +379,7 @@ private:
     std::vector<InputBuffer> inputs_;
     uint64_t image_bytes_ = 0;
     Stream stream_;
-    Event ev_[5];
+    Event ev_[4];  // start of prepare; end of prepare, scale and reduce
     uint64_t in_flight_ = 0;
     bool broken_ = false;  // a wait failed: every later call is refused
     std::array<float, 3> stage_ms_{};
