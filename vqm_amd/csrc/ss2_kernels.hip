@@ -1234,11 +1234,6 @@ __device__ __forceinline__ void unroll(std::integer_sequence<int, P...>, F&& f) 
     (f(std::integral_constant<int, P>{}), ...);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
-    return v;
-}
-
 // The six map values of one pixel from its blurred quantities `bl` (in the
 // form's order) and its raw samples a and b: d, d^4, ring, ring^4, blur,
 // blur^4 (scale.comp:305-333).
@@ -1561,49 +1556,59 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void sc
 
 // ---- reduce -----------------------------------------------------------------
 
-// One block per pair. Wave w takes the (level, channel) ranges w, w+16, ...
-// (18 at most, so nearly every range has a wave of its own and a single
-// pair's reduction is as long as its longest range, not the sum of four);
-// its lanes stride over the range's strips, each adding the six partial sums
-// of its strips in FP64 (four strips' loads in flight at a time, added in
-// strip order), and the wave then sums its lanes.
+// One block per (pair, level, channel): its threads stride over the range's
+// parts, each adding the six partial sums of its parts in FP64 (four parts'
+// loads in flight at a time), rows of 16 lanes and then six threads add them
+// up, and those write the six norms (zeros for a channel that is not stored).
+// Latency bound. A launch of one pair took 4.0 (96x64), 7.4 (1080p) and 11.4
+// us (4K) in one block of 16 waves a pair, a wave to a range; it takes 3.7, 3.9
+// and 5.3 (3.7 is an empty range's time). 8 pairs of 853x479: 5.8 -> 4.1 us;
+// 300 of 1080p: 16 -> 18, of 8,100 for all three kernels.
 // Norm level*18 + k: k < 6 is channel k/2's SSIM' slot k%2; k >= 6 is
 // channel (k-6)/4's edge slot 2 + (k-6)%4 (ring 1-, 4-norm, blur 1-, 4-norm).
-constexpr uint32_t kReduceWaves = 16;
+constexpr uint32_t kReduceThreads = 256;
+constexpr uint32_t kRanges = kMaxScales * kChannels;
 
-__global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const PairDesc* __restrict__ pairs) {
-    ConstAS<PairDesc>* pdp = as_const(pairs) + blockIdx.x;
+__global__ __launch_bounds__(kReduceThreads) void reduce_kernel(const PairDesc* __restrict__ pairs) {
+    __shared__ double rows[kReduceThreads / 16][6];
+    const uint32_t pair = blockIdx.x / kRanges, range = blockIdx.x % kRanges;
+    ConstAS<PairDesc>* pdp = as_const(pairs) + pair;
     ConstAS<Plan>* plan = as_const(pdp->plan);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    GlobalAS<const double>* partials = as_global(static_cast<const double*>(pdp->partials));
-    GlobalAS<double>* norms = as_global(pdp->norms);
-    for (uint32_t combo = wave; combo < static_cast<uint32_t>(kMaxScales * kChannels); combo += kReduceWaves) {
-        const uint32_t level = combo / kChannels, c = combo % kChannels;
-        const bool active = level < plan->levels && (plan->mask[level] & (1u << c)) != 0u;
+    const uint32_t level = range / kChannels, c = range % kChannels;
+    const bool active = level < plan->levels && (plan->mask[level] & (1u << c)) != 0u;
+    if (active) {
+        const uint32_t begin = plan->item_begin[level][c] << plan->part_shift;
+        const uint32_t count = plan->item_count[level][c] << plan->part_shift;
+        GlobalAS<const double>* p = as_global(static_cast<const double*>(pdp->partials)) +
+                                    static_cast<uint64_t>(begin) * 6u;
         double sum[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (active) {
-            const uint32_t begin = plan->item_begin[level][c] << plan->part_shift;
-            const uint32_t count = plan->item_count[level][c] << plan->part_shift;
 #pragma unroll 4
-            for (uint32_t it = lane; it < count; it += 64u) {
-                GlobalAS<const double>* p = partials + static_cast<uint64_t>(begin + it) * 6u;
+        for (uint32_t i = threadIdx.x; i < count; i += kReduceThreads)
 #pragma unroll
-                for (int k = 0; k < 6; ++k) sum[k] += p[k];
-            }
+            for (int k = 0; k < 6; ++k) sum[k] += p[static_cast<uint64_t>(i) * 6u + k];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) sum[k] = wave_sum(sum[k]);
+        for (int k = 0; k < 6; ++k) {
+            sum[k] = add_dpp<0xB1>(sum[k]);   // quad_perm [1, 0, 3, 2]
+            sum[k] = add_dpp<0x4E>(sum[k]);   // quad_perm [2, 3, 0, 1]
+            sum[k] = add_dpp<0x141>(sum[k]);  // row_half_mirror
+            sum[k] = add_dpp<0x140>(sum[k]);  // row_mirror
         }
-        if (lane != 0) continue;
-        const double one_per_pixel =
-            active ? 1.0 / (static_cast<double>(plan->w[level]) * static_cast<double>(plan->h[level])) : 0.0;
+        if (threadIdx.x % 16u == 0u)
 #pragma unroll
-        for (uint32_t slot = 0; slot < 6; ++slot) {
-            double value = one_per_pixel * sum[slot];
-            if (slot & 1u) value = sqrt(sqrt(value));
-            const uint32_t k = slot < 2u ? 2u * c + slot : 6u + 4u * c + (slot - 2u);
-            norms[level * 18u + k] = value;
-        }
+            for (int k = 0; k < 6; ++k) rows[threadIdx.x / 16u][k] = sum[k];
     }
+    __syncthreads();
+    const uint32_t slot = threadIdx.x;
+    if (slot >= 6u) return;
+    double value = 0.0;
+    if (active) {
+#pragma unroll
+        for (uint32_t r = 0; r < kReduceThreads / 16u; ++r) value += rows[r][slot];
+        value *= 1.0 / (static_cast<double>(plan->w[level]) * static_cast<double>(plan->h[level]));
+        if (slot & 1u) value = sqrt(sqrt(value));
+    }
+    const uint32_t k = slot < 2u ? 2u * c + slot : 6u + 4u * c + (slot - 2u);
+    as_global(pdp->norms)[level * 18u + k] = value;
 }
 
 // A plain streaming copy (16-byte loads and stores): the reference point that
@@ -1848,7 +1853,7 @@ hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const Pai
 
 hipError_t LaunchReduce(const PairDesc* pairs, uint32_t pairs_count, hipStream_t stream, hipEvent_t done) {
     if (pairs_count == 0) return Nothing(stream, done);
-    return Dispatch(&reduce_kernel, pairs_count, 64 * kReduceWaves, stream, done, pairs);
+    return Dispatch(&reduce_kernel, pairs_count * kRanges, kReduceThreads, stream, done, pairs);
 }
 
 }  // namespace vqm::ss2
