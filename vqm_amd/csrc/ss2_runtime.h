@@ -354,7 +354,8 @@ private:
     const InputBuffer& RequireBuffer(uint64_t handle, const char* name) const;
     // reuse_original: the original's planes are already in the workspace
     // (the resident reference cache), so only the distorted image is prepared.
-    uint64_t Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_original = false);
+    // uploaded: the sources were copied from host memory on the stream.
+    uint64_t Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_original = false, bool uploaded = false);
     void BuildGraph();
 
     vqm_ss2_config config_;
