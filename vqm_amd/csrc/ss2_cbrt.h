@@ -8,8 +8,11 @@
 //              second-order FP64 step from cbrt_fast's seed, rounded to
 //              FP32, with two exact FP64 comparisons for the one input in
 //              2^19 whose FP64 root lies too near a midpoint to round safely.
-//   cbrt_rn_near_hw, settled where `near` by cbrt_round_exact: the same root on the device from a hardware log2/exp2 seed
-//              and one FP64 step (the kernels' reference form).
+//   cbrt_rn_near_f32  the same root on the device in FP32 from a hardware
+//              log2/exp2 seed, on [2^-9, 2^15), but where it sets `near`: the
+//              kernels' reference form.
+//   cbrt_rn_near_hw   the same with one FP64 step, for every normal positive
+//              float: what those take with cbrt_round_exact.
 //
 // Every step of cbrt_fast and cbrt_rn is an IEEE conversion, add, multiply
 // or fused multiply-add (written out), with contraction off, so the result
@@ -103,7 +106,7 @@ __host__ __device__ inline float cbrt_rn_near(float x, bool* near) {
     return rounded;
 }
 
-// The seed of cbrt_rn_near_hw: x^(-1/3) as 2^(-log2(x) / 3) from the
+// The seed of the two roots below: x^(-1/3) as 2^(-log2(x) / 3) from the
 // hardware base-2 logarithm and exponential (v_log_f32, v_exp_f32; one
 // transcendental instruction each).
 __device__ inline float cbrt_seed_hw(float x) {
@@ -131,6 +134,37 @@ __device__ inline float cbrt_rn_near_hw(float x, bool* near) {
     const float rounded = static_cast<float>(y);
     const uint32_t dropped = static_cast<uint32_t>(__builtin_bit_cast(uint64_t, y)) & 0x1FFFFFFFu;
     *near = dropped - (0x10000000u - 0x200u) <= 2 * 0x200u;  // within 2^9 units of a midpoint
+    return rounded;
+}
+
+// The inputs cbrt_rn_near_f32 takes: bits from kCbrtF32First, this many.
+constexpr uint32_t kCbrtF32First = 0x3B000000u;                 // 2^-9
+constexpr uint32_t kCbrtF32Count = 0x47000000u - 0x3B000000u;  // up to 2^15
+
+// The root in FP32 operations. With s = x^(-1/3) (1 - h)^(1/3) from the
+// hardware seed and y = x s^2, the remainder R = x - y^3 is formed with one
+// rounding of its own size (y^2 = y2 + e2 exactly), and y + R s^2 / 3 is
+// within about 2 (2 h / 3)^2 of the root, relatively: at most 2.9e-5 of half
+// an ulp over [2^-9, 2^15), |h| <= 1.13e-6 (both measured there over every
+// float). The last fused multiply-add rounds that sum once, so the result is
+// the correctly rounded root unless the sum lies within 2^-14 of half an ulp
+// of a midpoint, which the test finds by moving it that much further: one
+// input in 16,000.
+// 15 instructions, 13 of them FP32 adds and multiplies (2.2 cycles) and two
+// transcendental (8.2), against 15 with six of FP64 (4.2) and three
+// conversions for cbrt_rn_near_hw.
+__device__ inline float cbrt_rn_near_f32(float x, bool* near) {
+    constexpr float kThird = 0x1.555556p-2f, kBeyond = 1.0f + 0x1p-14f;
+    const float s = cbrt_seed_hw(x);
+    const float s2 = s * s;
+    const float y = x * s2;
+    const float y2 = y * y;
+    const float e2 = __builtin_fmaf(y, y, -y2);
+    const float R = __builtin_fmaf(-e2, y, __builtin_fmaf(-y2, y, x));
+    const float inverse = s2 * kThird;
+    const float rounded = __builtin_fmaf(R, inverse, y);
+    const float rest = __builtin_fmaf(R, inverse, y - rounded);
+    *near = __builtin_fmaf(rest, kBeyond, rounded) != rounded;
     return rounded;
 }
 

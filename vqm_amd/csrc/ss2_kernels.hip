@@ -147,27 +147,39 @@ constexpr float kYOffset = 0.01f - kCbrtBias;  // rounded once
 // The cube roots of K mixes, in place. The reference form takes every root's
 // fast part first, so that the roots' instruction chains share a basic block
 // and interleave, and settles the rare near-midpoint roots in one branch for
-// all of them.
-template <bool Ref, int K>
+// all of them. Any: the mixes may be any positive normal float, else they lie
+// in cbrt_rn_near_f32's range.
+template <bool Ref, bool Any, int K>
 __device__ __forceinline__ void cube_roots(float (&m)[K]) {
     if constexpr (!Ref) {
 #pragma unroll
         for (int k = 0; k < K; ++k) m[k] = cbrt_fast(m[k]);
     } else {
         float c[K];
-        bool near = false;
+        bool unsettled[K], any = false;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            bool n;
-            c[k] = cbrt_rn_near_hw(m[k], &n);
-            near |= n;
+            c[k] = cbrt_rn_near_f32(m[k], &unsettled[k]);
+            if constexpr (Any) unsettled[k] |= __float_as_uint(m[k]) - kCbrtF32First >= kCbrtF32Count;
+            any |= unsettled[k];
         }
-        if (near) {
-            // Exact for every root, near or not: one copy of the code, the
-            // roots passing through it in turn.
+        if (any) {
+            // One copy of the exact root, the roots passing through it in
+            // turn; those that no lane has to settle pass by it.
+            uint32_t which = 0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) which |= (__builtin_amdgcn_ballot_w64(unsettled[k]) != 0u ? 1u : 0u) << k;
 #pragma unroll 1
             for (int k = 0; k < K; ++k) {
-                const float x = m[0], y = cbrt_round_exact(x, c[0]);
+                const float x = m[0];
+                float y = c[0];
+                if ((which >> k) & 1u) {
+                    if constexpr (Any) {
+                        bool n;
+                        y = cbrt_rn_near_hw(x, &n);
+                    }
+                    y = cbrt_round_exact(x, y);
+                }
 #pragma unroll
                 for (int i = 0; i + 1 < K; ++i) m[i] = m[i + 1], c[i] = c[i + 1];
                 m[K - 1] = x;
@@ -179,10 +191,10 @@ __device__ __forceinline__ void cube_roots(float (&m)[K]) {
     }
 }
 
-// Roots taken together: a lane's row of four pixels (two roots each).
-// Measured on 300 1080p pairs: 3.80 ms against 3.85 with two pixels' roots at
-// a time.
-constexpr int kRootBatch = 8;
+// Roots taken together: those of two pixels. Measured at 92 registers: one 4K
+// pair's prepare 38.5 us against 38.9 with four pixels' (94 registers, and
+// their `unsettled` masks spill).
+constexpr int kRootBatch = 4;
 
 // N pixels (px[j] = linear r, g, b): put(channel, values) for the channels in
 // `mask`. Clamp: the mixes may fall below the smallest normal float (samples
@@ -206,7 +218,7 @@ __device__ __forceinline__ void xyb_group(const float (*px)[3], uint32_t mask, P
         constexpr int n = sizeof(batch) / sizeof(float);
 #pragma unroll
         for (int i = 0; i < n; ++i) batch[i] = c[j + i];
-        cube_roots<Ref>(batch);
+        cube_roots<Ref, Clamp>(batch);
 #pragma unroll
         for (int i = 0; i < n; ++i) c[j + i] = batch[i];
     }
@@ -231,7 +243,7 @@ __device__ __forceinline__ void xyb_group(const float (*px)[3], uint32_t mask, P
         float b[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) b[j] = mix(px[j], kM20, kM21, kM22);
-        cube_roots<Ref>(b);
+        cube_roots<Ref, Clamp>(b);
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             const float sum = c[2 * j] + c[2 * j + 1];
@@ -968,7 +980,7 @@ __device__ __forceinline__ void prepare_coarse(ConstAS<Plan>* plan, GlobalAS<uin
                             fma_(k < 2u ? kM02 : kM22, v[2], kOpsinBias)))};
     static_assert(kM02 == kM12);
     if constexpr (Clamp) m[0] = fmaxf(m[0], kMinNormal);
-    cube_roots<Ref>(m);
+    cube_roots<Ref, Clamp>(m);
     lds.roots[lane] = Ref ? m[0] - kCbrtBias : m[0];
     wave_fence();
     // This lane's channel from its sample's roots.
@@ -1150,10 +1162,13 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
     prepare_coarse<Lay, Ref, General>(plan, planes, X0, Y0, lane, lds);
 }
 
-// What bounds it: VALU issue, of which the cube roots take over half (15
-// instructions each, six of FP64 at 4.2 cycles and two transcendentals at 8.2;
-// FP32 instructions take 2.2). 300 1080p pairs, reference form: 1.82e9 wave
-// instructions at 4.4 cycles each per SIMD.
+// What bounds it: VALU issue, of which the cube roots take about half (15
+// instructions each, two of them transcendentals at 8.2 cycles; FP32
+// instructions take 2.2). With the roots' last step in FP64 (six instructions
+// and three conversions at 4.2, values of two registers) and four waves a SIMD
+// 300 1080p pairs took 3.80 ms, one 4K pair 44.9 us; 3.56 ms and 41.8 us with
+// the FP32 step alone, 3.32 ms and 38.6 us with the fifth wave that its
+// registers leave room for (six waves, 80 registers, spill: 4.0 ms).
 //
 // A lane takes 4 x 4 base pixels, and with them the boxes of levels 1 and 2,
 // so that these need no exchange and every lane works at them; a pass over
@@ -1165,11 +1180,10 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
 // in the mixed form 0.90 -> 0.86 ms. A 96x64 pair, whose time is one wave's
 // chain of rows, takes 11.5 us against 9.8.
 //
-// Registers: 116 in the reference form (four waves a SIMD; at 96 the roots'
-// FP64 values spill), 91 in the difference form (five), 128 in the general
-// decode (four).
+// Registers: 92 in the reference form, 91 in the difference form (five waves
+// a SIMD), 128 in the general decode (four).
 template <typename Lay, bool General, bool Ref>
-__global__ __launch_bounds__(64 * kPrepWaves<General>) __attribute__((amdgpu_waves_per_eu(General || Ref ? 4 : 5))) void
+__global__ __launch_bounds__(64 * kPrepWaves<General>) __attribute__((amdgpu_waves_per_eu(General ? 4 : 5))) void
 prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ work, uint32_t tiles,
                uint32_t tiles_per_image, const float* __restrict__ lut_g, const uint8_t* src0, const uint8_t* src1) {
     constexpr uint32_t kWaves = kPrepWaves<General>, kHalves = kPrepTileH / kWaveRows;
@@ -1621,9 +1635,10 @@ __global__ __launch_bounds__(256) void copy_kernel(const uint4* __restrict__ src
 }
 
 // Self-check of the reference form's cube root over the floats with bits in
-// [first, end): cbrt_rn_near_hw settled by cbrt_round_exact (what the kernels take) against cbrt_rn (IEEE
-// steps only). Counts the inputs where they differ and those that took the
-// exact step, and keeps the smallest differing input and the largest
+// [first, end): cbrt_rn_near_hw settled by cbrt_round_exact, and on its range
+// cbrt_rn_near_f32 settled the same way, against cbrt_rn (IEEE steps only).
+// Counts the inputs where they differ and those where the FP64 step took the
+// exact one, and keeps the smallest differing input and the largest
 // |1 - x r^3| of the hardware seed r (as FP64 bits: non-negative doubles
 // order as their bits). One atomic per wave and counter.
 __global__ __launch_bounds__(256) void cbrt_check_kernel(uint32_t first, uint32_t end, CbrtCheck* out) {
@@ -1636,7 +1651,15 @@ __global__ __launch_bounds__(256) void cbrt_check_kernel(uint32_t first, uint32_
         const float rounded = cbrt_rn_near_hw(x, &n);
         const float got = n ? cbrt_round_exact(x, rounded) : rounded;
         near += n ? 1u : 0u;
-        if (got != cbrt_rn(x)) {
+        const float want = cbrt_rn(x);
+        bool differs = got != want;
+        if (static_cast<uint32_t>(u) - kCbrtF32First < kCbrtF32Count) {
+            bool unsettled;
+            float root = cbrt_rn_near_f32(x, &unsettled);
+            if (unsettled) root = cbrt_round_exact(x, root);
+            differs |= root != want;
+        }
+        if (differs) {
             ++bad;
             first_bad = min(first_bad, static_cast<uint32_t>(u));
         }
