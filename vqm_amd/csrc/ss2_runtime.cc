@@ -270,9 +270,12 @@ void WorkspacePools::Return(uint32_t width, uint32_t height, bool inputs, std::u
 
 namespace {
 // The event that ends a stage. It rides on the stage's kernel, or is recorded
-// behind it: for the order between two streams, and where images were uploaded
-// on the stream, whose next upload starts later behind a riding event (6 pairs
-// of 1080p from host memory over two pipelines: 1,606 us against 1,555).
+// behind it: for launches split over two streams, and where images were
+// uploaded on the stream, whose next upload starts later behind a riding event
+// (6 pairs of 1080p from host memory over two pipelines: 1,606 us against
+// 1,555). The runtime keeps a riding event's kernel until its stream is
+// synchronized or copies again: a lane's next launch does, with its
+// descriptors; Pipeline::Finish sees to it for pairs.
 struct StageEnd {
     StageEnd(const Event& event, hipStream_t stream, bool record)
         : rides(record ? nullptr : event.get()), recorded_(record ? event.get() : nullptr), stream_(stream) {}
@@ -424,6 +427,7 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
     const GeometryPlan& g0 = entries[0].plan->host;
     const PairDesc* dpairs = pairs_.as<PairDesc>();
     chunks_ = chunks;
+    const bool record = host_inputs || chunks > 1;
     for (uint32_t c = 0; c < chunks; ++c) {
         const uint32_t i0 = chunk_begin(c), i1 = chunk_begin(c + 1);
         // Uniform runs index pairs from their first descriptor; work lists
@@ -432,7 +436,7 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         const WorkRef* wp = uniform ? nullptr : wprep + prep_at[i0];
         const auto np = static_cast<uint32_t>(prep_at[i1] - prep_at[i0]);
         Check(hipEventRecord(Ev(4 * c).get(), s), "hipEventRecord");
-        const StageEnd prepared(Ev(4 * c + 1), s, host_inputs || chunks > 1);
+        const StageEnd prepared(Ev(4 * c + 1), s, record);
         Check(LaunchPrepare(fmt, map, general, base, wp, np, g0.prep_tiles, lut, nullptr, nullptr, s, persistent,
                             prepared.rides),
               "launch prepare");
@@ -443,13 +447,13 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         if (t != s) Check(hipStreamWaitEvent(t, Ev(4 * c + 1).get(), 0), "order scale after prepare");
         const auto ns = static_cast<uint32_t>(scale_at[i1] - scale_at[i0]);
         if (t != s) Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
-        const StageEnd scaled(Ev(4 * c + 3), t, host_inputs);
+        const StageEnd scaled(Ev(4 * c + 3), t, record);
         Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, uniform ? nullptr : wscale + scale_at[i0], ns,
                           g0.parts(), t, persistent, scaled.rides),
               "launch scale");
         scaled.Record();
     }
-    const StageEnd reduced(Ev(DoneEvent()), t, host_inputs);
+    const StageEnd reduced(Ev(DoneEvent()), t, record);
     Check(LaunchReduce(dpairs, count, t, reduced.rides), "launch reduce");
     reduced.Record();
     pending_ = true;
@@ -854,6 +858,11 @@ uint64_t Pipeline::SubmitBuffers(uint64_t a, uint64_t b, float background) {
     return Launch(base + ba.offset, base + bb.offset);
 }
 
+// The runtime keeps the kernels whose own dispatch sets an event (4.9 KB of
+// host memory a pair) until their stream is synchronized; a wait for the event
+// does not release them. Every 16th pair does: 2 us a pair, and 64 KB kept.
+constexpr uint32_t kSettlePairs = 16;
+
 uint32_t Pipeline::Finish(uint64_t token, double* norms) {
     if (token == 0 || token != in_flight_)
         Fail(VQM_INVALID_ARGUMENT, "unknown or already finished submission token");
@@ -870,6 +879,11 @@ uint32_t Pipeline::Finish(uint64_t token, double* norms) {
     else
         stage_ms_ = {Elapsed(ev_[0], ev_[1]), Elapsed(ev_[1], ev_[2]), Elapsed(ev_[2], ev_[3])};
     std::memcpy(norms, host_norms_.get(), kNorms * sizeof(double));
+    if (++settle_ % kSettlePairs == 0) {
+        const hipError_t settled = hipStreamSynchronize(stream_.get());
+        broken_ = settled != hipSuccess;
+        Check(settled, "settle the stream");
+    }
     return plan_.host.plan.levels;
 }
 

@@ -383,6 +383,7 @@ private:
     Event ev_[4];  // start of prepare; end of prepare, scale and reduce
     uint64_t in_flight_ = 0;
     bool broken_ = false;  // a wait failed: every later call is refused
+    uint32_t settle_ = 0;  // pairs finished
     std::array<float, 3> stage_ms_{};
     // Resident reference cache (vulkan.cc:238-241,716-735): the handle of
     // the resident original whose planes the workspace holds, or 0.
