@@ -34,6 +34,8 @@ inline constexpr uint32_t kDefaultStripCols = 128;
 constexpr bool ValidStripCols(uint32_t cols) { return cols == 64 || cols == 128; }
 // Strip heights are multiples of the map-sum block height (8 rows).
 inline constexpr uint32_t kSumBlockRows = 8;
+// Output rows of a block of the scale kernel's block form.
+inline constexpr uint32_t kBlockRows = 32;
 // Plane padding: 6 zero rows above, 8 zero columns on the left (so rows of
 // four samples stay 16-byte aligned), and enough on the right and below to
 // cover the last strip's halo.

@@ -226,6 +226,8 @@ void PackView(const vqm_host_view& view, uint8_t* dst) {
 Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
               uint32_t row_parts) {
     const ScalePlan scales = PlanScales(width, height);
+    const bool block_form = row_parts == 0;
+    if (block_form) strip_rows = kBlockRows, strip_cols = 64, row_parts = 1;
     if (strip_rows == 0) strip_rows = 64;
     if (strip_cols == 0) strip_cols = kDefaultStripCols;
     if (strip_rows % kSumBlockRows != 0 || strip_rows > 1024)
@@ -253,7 +255,8 @@ Plan FillPlan(uint32_t width, uint32_t height, PlaneFormat format, uint32_t stri
         const uint32_t strips = (p.w[l] + kStripCols - 1) / kStripCols;
         const uint32_t bands = (p.h[l] + strip_rows - 1) / strip_rows;
         p.pitch[l] = static_cast<uint32_t>(Align(static_cast<uint64_t>(strips) * kStripCols + 14, 4));
-        p.rows[l] = bands * strip_rows + 2 * kRadius;
+        // Whole strips; a block reads no row past its last output row's.
+        p.rows[l] = (block_form ? static_cast<uint32_t>(Align(p.h[l], kSumBlockRows)) : bands * strip_rows) + 2 * kRadius;
         for (uint32_t c = 0; c < static_cast<uint32_t>(kChannels); ++c) {
             if (ChannelPruned(c, l, scales.count)) continue;
             p.mask[l] |= 1u << c;
@@ -335,6 +338,14 @@ uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t 
 
 uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                             uint32_t strip_cols) {
+    // Blocks up to the count where the two forms' scale launches met, measured
+    // on one pair of 8x8 to 4K: FP32 planes at 3440x1900 (5,400 blocks: 62.7 us
+    // against 61.6; 1080p, 1,752: 23.2 against 27.2; 96x64 5.9 against 10.2),
+    // 16-bit planes, whose samples a block converts four times, from 1080p on
+    // (FP16 25.8 against 27.4, the pair's time equal; 2560x1440 44.4 against
+    // 41.3).
+    const uint64_t most = (ElementBytes(format) == 4 ? 20 : 6) * static_cast<uint64_t>(kWholeDeviceCUs);
+    if (strip_rows == 0 && strip_cols == 0 && FillPlan(width, height, format, 0, 0, 0).items <= most) return 0;
     return strip_rows != 0 ? 1
                            : RowParts(width, height, format,
                                       SinglePairStripRows(width, height, format, 0, strip_cols), strip_cols, 1,
@@ -350,6 +361,7 @@ GeometryPlan BuildPlan(uint32_t width, uint32_t height, PlaneFormat format, uint
                        uint32_t strip_cols, uint32_t row_parts) {
     GeometryPlan g;
     g.plan = FillPlan(width, height, format, strip_rows, strip_cols, row_parts);
+    g.block_form = row_parts == 0;
     g.format = format;
     g.plane_bytes_per_image = g.plan.image_bytes;
     g.prep_tiles = g.plan.prep_tiles_x * g.plan.prep_tiles_y;

@@ -75,13 +75,16 @@ struct GeometryPlan {
     uint64_t plane_bytes_per_image = 0;  // padded plane storage
     PlaneFormat format = kPlaneF32;
     uint32_t prep_tiles = 0;             // prepare blocks per image
+    bool block_form = false;             // the scale kernel's form (RowParts)
     uint32_t parts() const { return plan.items << plan.part_shift; }  // scale blocks per pair
 };
 
 // strip_rows: output rows per scale work item, a multiple of 8 up to 1024
 // (0 = 64; launches pick theirs with DefaultStripRows); strip_cols: its
 // width, 64 or 128 columns (0 = 128); row_parts: 1, 2 or 4 bands of a
-// multiple of 8 rows a strip is cut into, one wave each (RowParts).
+// multiple of 8 rows a strip is cut into, one wave each (RowParts), or 0: the
+// scale kernel's block form, whose strips are kBlockRows rows by 64 columns
+// whatever the other two are.
 GeometryPlan BuildPlan(uint32_t width, uint32_t height, PlaneFormat format,
                        uint32_t strip_rows, uint32_t strip_cols = 0, uint32_t row_parts = 1);
 
@@ -118,7 +121,8 @@ uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t 
                   uint64_t pairs, uint32_t cus);
 
 // RowParts of a single-pair pipeline's default height (of the geometry
-// alone, as SinglePairStripRows); 1 when `strip_rows` is set.
+// alone, as SinglePairStripRows), or 0 for the block form, where neither
+// `strip_rows` nor `strip_cols` is set; 1 when `strip_rows` is set.
 uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                             uint32_t strip_cols);
 

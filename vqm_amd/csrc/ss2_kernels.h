@@ -43,10 +43,11 @@ hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const Pa
 // work = nullptr; else work[].index is a part. `blur` picks the kernel: kBlurSampled (13-tap sampled Gaussian)
 // or kBlurRecursive (the recursive Gaussian's 9-tap truncated-cosine
 // kernel); `map` the SSIM' map's form, which must be the one the planes were
-// prepared with.
+// prepared with. block_form: the plans are of that form (GeometryPlan), a
+// block of 512 threads per item; uniform launches only.
 hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
-                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent = false,
-                       hipEvent_t done = nullptr);
+                       uint32_t blocks, uint32_t parts_per_pair, bool block_form, hipStream_t stream,
+                       bool persistent = false, hipEvent_t done = nullptr);
 
 // Sums each (level, channel) norm's partials in FP64 and writes the 108 norms
 // (device or pinned host memory).

@@ -267,6 +267,7 @@ struct F32 {
     static __device__ __forceinline__ void unpack4(Raw4 v, float out[4]) {
         for (int i = 0; i < 4; ++i) out[i] = v[i];
     }
+    static __device__ __forceinline__ float load1(GlobalAS<const E>* p) { return *p; }
     static __device__ __forceinline__ void store1(GlobalAS<E>* p, float v) { *p = v; }
     static __device__ __forceinline__ void store2(GlobalAS<E>* p, float a, float b) {
         *reinterpret_cast<GlobalAS<f32x2>*>(p) = f32x2{a, b};
@@ -317,6 +318,7 @@ struct Narrow {
             out[2 * i + 1] = From(static_cast<uint16_t>(v[i] >> 16));
         }
     }
+    static __device__ __forceinline__ float load1(GlobalAS<const E>* p) { return From(*p); }
     static __device__ __forceinline__ void store1(GlobalAS<E>* p, float v) { *p = To(v); }
     static __device__ __forceinline__ void store2(GlobalAS<E>* p, float a, float b) {
         *reinterpret_cast<GlobalAS<uint32_t>*>(p) =
@@ -1298,6 +1300,38 @@ __device__ __forceinline__ void map_values(const float* bl, float a, float b, fl
     v6[5] = bb * bb;
 }
 
+// Adds source columns 4 t .. 4 t + 3 of a row (samples a, b of both images) to
+// the horizontal sums of its output columns 0 .. 3, whose taps ascend with the
+// source column (scale.comp:187-241).
+template <typename TapsT, bool Ref>
+__device__ __forceinline__ void blur_quad(int t, f32x4 a, f32x4 b, float (&acc)[kBlurred<Ref>][4]) {
+    constexpr int Q = kBlurred<Ref>;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int m = 4 * t + e;
+        const float x = a[e], y = b[e];
+        float v[Q];
+        v[0] = x;
+        v[1] = y;
+        if constexpr (Ref) {
+            v[2] = x * x;
+            v[3] = y * y;
+            v[4] = x * y;
+        } else {
+            const float d = x - y;
+            v[2] = d * d;
+            v[3] = x * y;
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int k = m - c;
+                if (k == 0) acc[q][c] = TapsT::w[0] * v[q];
+                if (k > 0 && k < kTaps) acc[q][c] = fma_(TapsT::w[k], v[q], acc[q][c]);
+            }
+    }
+}
 
 // One wave's LDS: the raw rows of the last kRawSlots steps, and the
 // exchange that turns horizontal results (lane = row and column group) into
@@ -1394,31 +1428,7 @@ __device__ __forceinline__ void scale_strip(ConstAS<PairDesc>* pdp, ConstAS<Plan
                     na = *reinterpret_cast<const f32x4*>(ra + 4 * t + 4);
                     nb = *reinterpret_cast<const f32x4*>(rb + 4 * t + 4);
                 }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int m = 4 * t + e;
-                    const float x = va[e], y = vb[e];
-                    float v[Q];
-                    v[0] = x;
-                    v[1] = y;
-                    if constexpr (Ref) {
-                        v[2] = x * x;
-                        v[3] = y * y;
-                        v[4] = x * y;
-                    } else {
-                        const float d = x - y;
-                        v[2] = d * d;
-                        v[3] = x * y;
-                    }
-#pragma unroll
-                    for (int q = 0; q < Q; ++q)
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            const int k = m - c;
-                            if (k == 0) acc[q][c] = TapsT::w[0] * v[q];
-                            if (k > 0 && k < kTaps) acc[q][c] = fma_(TapsT::w[k], v[q], acc[q][c]);
-                        }
-                }
+                blur_quad<TapsT, Ref>(t, va, vb, acc);
                 va = na;
                 vb = nb;
                 __builtin_amdgcn_sched_barrier(0);
@@ -1565,6 +1575,156 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void sc
         }
         GlobalAS<double>* out = as_global(pdp->partials) + static_cast<uint64_t>(part) * 6u;
         if (lane < 48u && (lane & 7u) == 0u) out[lane >> 3] = v;
+    }
+}
+
+// The block form of the scale kernel, for launches of few pairs, whose time is
+// the chain of one wave's steps: a block of eight waves takes 64 columns by 32
+// rows of a level and channel.
+//
+// The waves blur the block's 44 source rows horizontally, four rows a wave at
+// a time as above but from global memory, into LDS; after a barrier each takes
+// 8 rows of 32 columns, a lane four rows of a column, down the columns. So a
+// wave's chain is one or two horizontal passes and four output rows' vertical
+// ones, against five and more steps of both, and the 12 rows above a band are
+// blurred once for 32 output rows, not once for each 8 or 16.
+//
+// What bounds it: at 96x64 that chain, some 10,000 cycles against 22,900 (2,000
+// of them the reads of the descriptor, the plan and the item); from 1080p on
+// VALU issue. One pair's launch, reference form: 96x64 10.2 -> 5.9 us, 512x512
+// 11.7 -> 6.6, 1080p 27.2 -> 23.2, 2560x1440 41.2 -> 38.4; a 4K pair takes 77
+// against 71 us (SinglePairRowParts). 78 registers and 69,888 bytes of LDS: two
+// blocks a CU.
+constexpr int kBlockWaves = 8;
+constexpr int kBlockSourceRows = static_cast<int>(kBlockRows) + 2 * kRadius;
+constexpr int kBlockPitch = 72;  // floats a row: rows four apart lie 32 banks apart
+
+template <bool Ref>
+struct BlockLds {
+    float blurred[kBlurred<Ref>][kBlockSourceRows][kBlockPitch];
+    float sums[kBlockWaves][6][32];
+    double parts[kBlockWaves][6];
+};
+
+template <typename Lay, typename TapsT, bool Ref>
+__global__ __launch_bounds__(64 * kBlockWaves) __attribute__((amdgpu_waves_per_eu(4))) void scale_block_kernel(
+    const PairDesc* __restrict__ pairs, uint32_t blocks, uint32_t items_per_pair) {
+    using Fmt = typename Lay::Fmt;
+    using E = typename Fmt::E;
+    constexpr int Q = kBlurred<Ref>;
+    __shared__ __align__(16) BlockLds<Ref> lds;
+    const uint32_t l = xcd_remap(blockIdx.x, blocks);
+    const uint32_t pair_idx = l / items_per_pair, index = l - pair_idx * items_per_pair;
+    ConstAS<PairDesc>* pdp = as_const(pairs) + pair_idx;
+    ConstAS<Plan>* plan = as_const(pdp->plan);
+    ConstAS<ScaleItem>* item = as_const(pdp->items) + index;
+    const uint32_t level = item->level, channel = item->channel, x0 = item->x0, y0 = item->y0;
+    const uint32_t W = plan->w[level], pitch = plan->pitch[level];
+    const int out = static_cast<int>(min(kBlockRows, plan->h[level] - y0));  // the level ends below them
+    const int total = out + 2 * kRadius, units = (total + kStep - 1) / kStep;
+    const int wave = static_cast<int>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63u;
+
+    // Source row r is padded row y0 + r, source column j is padded x0 + 2 + j
+    // (as in scale_strip).
+    GlobalAS<const uint8_t>* base = as_global(static_cast<const uint8_t*>(pdp->planes)) +
+                                    plan->plane_off[level][channel] +
+                                    (static_cast<uint64_t>(y0) * pitch + x0 + 2u) * sizeof(E);
+    GlobalAS<const E>* pa = reinterpret_cast<GlobalAS<const E>*>(base);
+    GlobalAS<const E>* pb = reinterpret_cast<GlobalAS<const E>*>(base + plan->image_bytes);
+
+    // Vertical role: lane = four rows from row0 of column `col`; its own
+    // samples are loaded ahead (rows past the block's last are that row).
+    const int row0 = 8 * (wave >> 1) + 4 * static_cast<int>(lane >> 5);
+    const uint32_t col = 32u * (static_cast<uint32_t>(wave) & 1u) + (lane & 31u);
+    float own[kStep][2];
+#pragma unroll
+    for (int j = 0; j < kStep; ++j) {
+        const uint32_t at = static_cast<uint32_t>(min(row0 + j, out - 1) + kRadius) * pitch + kRadius + col;
+        own[j][0] = Fmt::load1(pa + at);
+        own[j][1] = Fmt::load1(pb + at);
+    }
+
+    for (int unit = wave; unit < units; unit += kBlockWaves) {
+        const uint32_t r = static_cast<uint32_t>(unit) * kStep + (lane >> 4), g = lane & 15u;
+        const uint32_t at = r * pitch + 4u * g;
+        typename Fmt::Raw4 ra[4], rb[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            ra[t] = Fmt::load4(pa + at + 4 * t);
+            rb[t] = Fmt::load4(pb + at + 4 * t);
+        }
+        float acc[Q][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            float a[4], b[4];
+            Fmt::unpack4(ra[t], a);
+            Fmt::unpack4(rb[t], b);
+            blur_quad<TapsT, Ref>(t, f32x4{a[0], a[1], a[2], a[3]}, f32x4{b[0], b[1], b[2], b[3]}, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            *reinterpret_cast<f32x4*>(&lds.blurred[q][r][4u * g]) = f32x4{acc[q][0], acc[q][1], acc[q][2], acc[q][3]};
+    }
+    __syncthreads();
+
+    double v = 0.0;
+    if (8 * (wave >> 1) < out) {
+        // Taps ascend with the source row (scale.comp:243-298).
+        float done[kStep][Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+#pragma unroll
+            for (int m = 0; m < kTaps - 1 + kStep; ++m) {
+                const float h = lds.blurred[q][row0 + m][col];
+#pragma unroll
+                for (int j = 0; j < kStep; ++j) {
+                    const int k = m - j;
+                    if (k == 0) done[j][q] = TapsT::w[0] * h;
+                    if (k > 0 && k < kTaps) done[j][q] = fma_(TapsT::w[k], h, done[j][q]);
+                }
+            }
+        }
+        // FP32 sums of the level's rows 8 k .. 8 k + 7 in their order: the
+        // lower lanes' four rows, then the upper lanes'.
+        float v6[kStep][6], sum[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < kStep; ++j) {
+            map_values<Ref>(done[j], own[j][0], own[j][1], v6[j]);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                v6[j][k] = row0 + j < out ? v6[j][k] : 0.0f;
+                sum[k] = sum[k] + v6[j][k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            sum[k] = __int_as_float(
+                __builtin_amdgcn_ds_bpermute(static_cast<int>(4u * (lane & 31u)), __float_as_int(sum[k])));
+#pragma unroll
+            for (int j = 0; j < kStep; ++j) sum[k] = sum[k] + v6[j][k];
+            if (lane >= 32u) lds.sums[wave][k][lane - 32u] = sum[k];
+        }
+        wave_fence();
+        // Lanes 8 k .. 8 k + 7 add map k's columns that lie in the level.
+        const uint32_t k = min(lane >> 3, 5u);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t c = (lane & 7u) + 8u * i;
+            v += x0 + 32u * (static_cast<uint32_t>(wave) & 1u) + c < W ? static_cast<double>(lds.sums[wave][k][c]) : 0.0;
+        }
+        v = add_dpp<0xB1>(v);
+        v = add_dpp<0x4E>(v);
+        v = add_dpp<0x141>(v);
+    }
+    if (lane < 48u && (lane & 7u) == 0u) lds.parts[wave][lane >> 3] = v;
+    __syncthreads();
+    if (threadIdx.x < 6u) {
+        double total_k = 0.0;
+#pragma unroll
+        for (int w = 0; w < kBlockWaves; ++w) total_k += lds.parts[w][threadIdx.x];
+        as_global(pdp->partials)[static_cast<uint64_t>(index) * 6u + threadIdx.x] = total_k;
     }
 }
 
@@ -1789,25 +1949,28 @@ hipError_t launch_prepare_t(MapForm map, bool general, const PairDesc* pairs, co
 
 template <typename Lay, typename TapsT, bool Ref>
 hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t parts,
-                          bool persistent, hipStream_t stream, hipEvent_t done) {
+                          bool block_form, bool persistent, hipStream_t stream, hipEvent_t done) {
+    if (block_form)
+        return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, blocks, 64 * kBlockWaves, stream, done, pairs, blocks,
+                        parts);
     const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref>, 64, blocks, persistent);
     return Dispatch(&scale_kernel<Lay, TapsT, Ref>, grid, 64, stream, done, pairs, work, blocks, parts);
 }
 
 template <typename Lay, bool Ref>
 hipError_t launch_scale_m(uint32_t blur, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
-                          uint32_t parts, bool persistent, hipStream_t stream, hipEvent_t done) {
+                          uint32_t parts, bool block_form, bool persistent, hipStream_t stream, hipEvent_t done) {
     return blur == kBlurRecursive
-               ? launch_scale_g<Lay, CosineTaps, Ref>(pairs, work, blocks, parts, persistent, stream, done)
-               : launch_scale_g<Lay, SampledTaps, Ref>(pairs, work, blocks, parts, persistent, stream, done);
+               ? launch_scale_g<Lay, CosineTaps, Ref>(pairs, work, blocks, parts, block_form, persistent, stream, done)
+               : launch_scale_g<Lay, SampledTaps, Ref>(pairs, work, blocks, parts, block_form, persistent, stream, done);
 }
 
 template <typename Lay>
 hipError_t launch_scale_t(uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work, uint32_t blocks,
-                          uint32_t parts, bool persistent, hipStream_t stream, hipEvent_t done) {
+                          uint32_t parts, bool block_form, bool persistent, hipStream_t stream, hipEvent_t done) {
     return map == kMapReference
-               ? launch_scale_m<Lay, true>(blur, pairs, work, blocks, parts, persistent, stream, done)
-               : launch_scale_m<Lay, false>(blur, pairs, work, blocks, parts, persistent, stream, done);
+               ? launch_scale_m<Lay, true>(blur, pairs, work, blocks, parts, block_form, persistent, stream, done)
+               : launch_scale_m<Lay, false>(blur, pairs, work, blocks, parts, block_form, persistent, stream, done);
 }
 
 }  // namespace
@@ -1860,16 +2023,21 @@ hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const Pa
 }
 
 hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
-                       uint32_t blocks, uint32_t parts_per_pair, hipStream_t stream, bool persistent,
-                       hipEvent_t done) {
+                       uint32_t blocks, uint32_t parts_per_pair, bool block_form, hipStream_t stream,
+                       bool persistent, hipEvent_t done) {
     if (blocks == 0) return Nothing(stream, done);
+    if (block_form && (work != nullptr || persistent)) return hipErrorInvalidValue;
     if (blur > kBlurRecursive || map > kMapDifference) return hipErrorInvalidValue;
     const uint32_t n = parts_per_pair;
     switch (format) {
-        case kPlaneF32: return launch_scale_t<LayoutF32>(blur, map, pairs, work, blocks, n, persistent, stream, done);
-        case kPlaneF16: return launch_scale_t<LayoutF16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
-        case kPlaneBF16: return launch_scale_t<LayoutBF16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
-        case kPlaneU16: return launch_scale_t<LayoutU16>(blur, map, pairs, work, blocks, n, persistent, stream, done);
+        case kPlaneF32:
+            return launch_scale_t<LayoutF32>(blur, map, pairs, work, blocks, n, block_form, persistent, stream, done);
+        case kPlaneF16:
+            return launch_scale_t<LayoutF16>(blur, map, pairs, work, blocks, n, block_form, persistent, stream, done);
+        case kPlaneBF16:
+            return launch_scale_t<LayoutBF16>(blur, map, pairs, work, blocks, n, block_form, persistent, stream, done);
+        case kPlaneU16:
+            return launch_scale_t<LayoutU16>(blur, map, pairs, work, blocks, n, block_form, persistent, stream, done);
     }
     return hipErrorInvalidValue;
 }

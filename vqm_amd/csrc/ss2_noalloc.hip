@@ -124,11 +124,13 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
     // The strip height a pipeline of this geometry takes, so both give the
     // same sums.
     SetupArgs args{};
+    const uint32_t row_parts =
+        SinglePairRowParts(config.width, config.height, format, config.strip_rows, config.strip_cols);
     args.plan = FillPlan(config.width, config.height, format,
                          SinglePairStripRows(config.width, config.height, format, config.strip_rows,
                                              config.strip_cols),
                          config.strip_cols,
-                         SinglePairRowParts(config.width, config.height, format, config.strip_rows, config.strip_cols));
+                         row_parts);
     const Plan& p = args.plan;
     const uint64_t parts = static_cast<uint64_t>(p.items) << p.part_shift;
     const uint64_t partials_at = Align256(kItemsAt + static_cast<uint64_t>(p.items) * sizeof(ScaleItem));
@@ -164,7 +166,7 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
     Check(LaunchPrepare(format, map, false, dpair, nullptr, 2 * tiles, tiles, dlut, nullptr, nullptr, stream),
           "launch prepare");
     Check(LaunchScale(format, config.blur, map, dpair, nullptr, static_cast<uint32_t>(parts), static_cast<uint32_t>(parts),
-                      stream),
+                      row_parts == 0, stream),
           "launch scale");
     Check(LaunchReduce(dpair, 1, stream), "launch reduce");
     return p.levels;

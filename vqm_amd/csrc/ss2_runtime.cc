@@ -320,7 +320,7 @@ hipGraphExec_t Lane::CaptureGraph(PlaneFormat fmt, MapForm map, const float* lut
         e = LaunchPrepare(fmt, map, false, dpairs, nullptr, static_cast<uint32_t>(prep), g.prep_tiles, lut, nullptr,
                           nullptr, s, persistent);
     if (e == hipSuccess)
-        e = LaunchScale(fmt, blur, map, dpairs, nullptr, static_cast<uint32_t>(scale), g.parts(), s, persistent);
+        e = LaunchScale(fmt, blur, map, dpairs, nullptr, static_cast<uint32_t>(scale), g.parts(), g.block_form, s, persistent);
     if (e == hipSuccess) e = LaunchReduce(dpairs, count, s);
     hipGraph_t graph = nullptr;
     const hipError_t end = hipStreamEndCapture(s, &graph);
@@ -449,7 +449,7 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         if (t != s) Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
         const StageEnd scaled(Ev(4 * c + 3), t, record);
         Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, uniform ? nullptr : wscale + scale_at[i0], ns,
-                          g0.parts(), t, persistent, scaled.rides),
+                          g0.parts(), g0.block_form, t, persistent, scaled.rides),
               "launch scale");
         scaled.Record();
     }
@@ -611,7 +611,7 @@ void Pipeline::BuildGraph() {
     if (e == hipSuccess)
         e = LaunchPrepare(fmt, map_, false, pd, nullptr, 2 * g.prep_tiles, g.prep_tiles, ctx_.lut, nullptr, nullptr, s);
     if (e == hipSuccess)
-        e = LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s);
+        e = LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), g.block_form, s);
     if (e == hipSuccess) e = LaunchReduce(pd, 1, s);
     hipGraph_t graph = nullptr;
     const hipError_t end = hipStreamEndCapture(s, &graph);
@@ -701,7 +701,7 @@ uint64_t Pipeline::Launch(const uint8_t* src0, const uint8_t* src1, bool reuse_o
                               s, false, prepared.rides),
           "launch prepare");
     prepared.Record();
-    Check(LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), s, false, scaled.rides),
+    Check(LaunchScale(fmt, config_.blur, map_, pd, nullptr, g.parts(), g.parts(), g.block_form, s, false, scaled.rides),
           "launch scale");
     scaled.Record();
     Check(LaunchReduce(pd, 1, s, reduced.rides), "launch reduce");
