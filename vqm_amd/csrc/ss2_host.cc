@@ -336,16 +336,20 @@ uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t 
     return best;
 }
 
+bool PrefersBlocks(uint32_t width, uint32_t height, PlaneFormat format, uint64_t pairs, uint32_t cus) {
+    // Up to the count of blocks where the two forms' scale launches met,
+    // measured on one pair of 8x8 to 4K: FP32 planes at 3440x1900 (5,400 blocks:
+    // 62.7 us against 61.6; 1080p, 1,752: 23.2 against 27.2; 96x64 5.9 against
+    // 10.2), 16-bit planes, whose samples a block converts four times, from
+    // 1080p on (FP16 25.8 against 27.4, the pair's time equal; 2560x1440 44.4
+    // against 41.3).
+    const uint64_t most = (ElementBytes(format) == 4 ? 20 : 6) * static_cast<uint64_t>(cus);
+    return FillPlan(width, height, format, 0, 0, 0).items * pairs <= most;
+}
+
 uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                             uint32_t strip_cols) {
-    // Blocks up to the count where the two forms' scale launches met, measured
-    // on one pair of 8x8 to 4K: FP32 planes at 3440x1900 (5,400 blocks: 62.7 us
-    // against 61.6; 1080p, 1,752: 23.2 against 27.2; 96x64 5.9 against 10.2),
-    // 16-bit planes, whose samples a block converts four times, from 1080p on
-    // (FP16 25.8 against 27.4, the pair's time equal; 2560x1440 44.4 against
-    // 41.3).
-    const uint64_t most = (ElementBytes(format) == 4 ? 20 : 6) * static_cast<uint64_t>(kWholeDeviceCUs);
-    if (strip_rows == 0 && strip_cols == 0 && FillPlan(width, height, format, 0, 0, 0).items <= most) return 0;
+    if (strip_rows == 0 && strip_cols == 0 && PrefersBlocks(width, height, format, 1, kWholeDeviceCUs)) return 0;
     return strip_rows != 0 ? 1
                            : RowParts(width, height, format,
                                       SinglePairStripRows(width, height, format, 0, strip_cols), strip_cols, 1,

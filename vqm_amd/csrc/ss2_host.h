@@ -120,6 +120,10 @@ uint32_t SinglePairStripRows(uint32_t width, uint32_t height, PlaneFormat format
 uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows, uint32_t strip_cols,
                   uint64_t pairs, uint32_t cus);
 
+// Whether a scale launch of `pairs` pairs of this geometry alone takes the
+// block form.
+bool PrefersBlocks(uint32_t width, uint32_t height, PlaneFormat format, uint64_t pairs, uint32_t cus);
+
 // RowParts of a single-pair pipeline's default height (of the geometry
 // alone, as SinglePairStripRows), or 0 for the block form, where neither
 // `strip_rows` nor `strip_cols` is set; 1 when `strip_rows` is set.

@@ -44,7 +44,7 @@ hipError_t LaunchPrepare(PlaneFormat format, MapForm map, bool general, const Pa
 // or kBlurRecursive (the recursive Gaussian's 9-tap truncated-cosine
 // kernel); `map` the SSIM' map's form, which must be the one the planes were
 // prepared with. block_form: the plans are of that form (GeometryPlan), a
-// block of 512 threads per item; uniform launches only.
+// block of 512 threads per item; not with `persistent`.
 hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const PairDesc* pairs, const WorkRef* work,
                        uint32_t blocks, uint32_t parts_per_pair, bool block_form, hipStream_t stream,
                        bool persistent = false, hipEvent_t done = nullptr);

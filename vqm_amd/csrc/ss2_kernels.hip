@@ -1608,13 +1608,21 @@ struct BlockLds {
 
 template <typename Lay, typename TapsT, bool Ref>
 __global__ __launch_bounds__(64 * kBlockWaves) __attribute__((amdgpu_waves_per_eu(4))) void scale_block_kernel(
-    const PairDesc* __restrict__ pairs, uint32_t blocks, uint32_t items_per_pair) {
+    const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ work, uint32_t blocks, uint32_t items_per_pair) {
     using Fmt = typename Lay::Fmt;
     using E = typename Fmt::E;
     constexpr int Q = kBlurred<Ref>;
     __shared__ __align__(16) BlockLds<Ref> lds;
     const uint32_t l = xcd_remap(blockIdx.x, blocks);
-    const uint32_t pair_idx = l / items_per_pair, index = l - pair_idx * items_per_pair;
+    uint32_t pair_idx, index;
+    if (work != nullptr) {
+        ConstAS<WorkRef>* w = as_const(work) + l;
+        pair_idx = w->pair;
+        index = w->index;
+    } else {
+        pair_idx = l / items_per_pair;
+        index = l - pair_idx * items_per_pair;
+    }
     ConstAS<PairDesc>* pdp = as_const(pairs) + pair_idx;
     ConstAS<Plan>* plan = as_const(pdp->plan);
     ConstAS<ScaleItem>* item = as_const(pdp->items) + index;
@@ -1951,8 +1959,8 @@ template <typename Lay, typename TapsT, bool Ref>
 hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t parts,
                           bool block_form, bool persistent, hipStream_t stream, hipEvent_t done) {
     if (block_form)
-        return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, blocks, 64 * kBlockWaves, stream, done, pairs, blocks,
-                        parts);
+        return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, blocks, 64 * kBlockWaves, stream, done, pairs, work,
+                        blocks, parts);
     const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref>, 64, blocks, persistent);
     return Dispatch(&scale_kernel<Lay, TapsT, Ref>, grid, 64, stream, done, pairs, work, blocks, parts);
 }
@@ -2026,7 +2034,7 @@ hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const Pai
                        uint32_t blocks, uint32_t parts_per_pair, bool block_form, hipStream_t stream,
                        bool persistent, hipEvent_t done) {
     if (blocks == 0) return Nothing(stream, done);
-    if (block_form && (work != nullptr || persistent)) return hipErrorInvalidValue;
+    if (block_form && persistent) return hipErrorInvalidValue;
     if (blur > kBlurRecursive || map > kMapDifference) return hipErrorInvalidValue;
     const uint32_t n = parts_per_pair;
     switch (format) {

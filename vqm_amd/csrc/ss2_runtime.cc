@@ -341,7 +341,10 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
     auto* hp = h_pairs_.as<PairDesc>();
     bool uniform = true, general = false;
     uint64_t prep_work = 0, scale_work = 0;
-    std::vector<uint64_t> prep_at(count + 1, 0), scale_at(count + 1, 0);  // work-list offsets
+    // Work-list offsets; scale_at[1]: of the pairs whose plans have the block
+    // form, behind all the others'.
+    std::vector<uint64_t> prep_at(count + 1, 0), scale_at[2];
+    for (auto& at : scale_at) at.assign(count + 1, 0);
     for (uint32_t i = 0; i < count; ++i) {
         const LaunchEntry& e = entries[i];
         PairDesc& pd = hp[i];
@@ -359,7 +362,8 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         prep_work += 2ull * e.plan->host.prep_tiles;
         scale_work += e.plan->host.parts();
         prep_at[i + 1] = prep_work;
-        scale_at[i + 1] = scale_work;
+        for (bool form : {false, true})
+            scale_at[form][i + 1] = scale_at[form][i] + (e.plan->host.block_form == form ? e.plan->host.parts() : 0);
     }
     if (prep_work > 0x7FFFFFFFull || scale_work > 0x7FFFFFFFull)
         Fail(VQM_INVALID_ARGUMENT, "the submission has too many work items");
@@ -410,16 +414,19 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
         }
         auto* wp = h_work_prep_.as<WorkRef>();
         auto* ws = h_work_scale_.as<WorkRef>();
-        uint64_t np = 0, ns = 0;
+        uint64_t np = 0, ns[2] = {0, scale_at[0][count]};
         for (uint32_t i = 0; i < count; ++i) {
             const GeometryPlan& g = entries[i].plan->host;
             for (uint32_t image = 0; image < 2; ++image)
                 for (uint32_t k = 0; k < g.prep_tiles; ++k) wp[np++] = WorkRef{i, k | (image << 31)};
-            for (uint32_t k = 0; k < g.parts(); ++k) ws[ns++] = WorkRef{i, k};
+            const uint32_t parts = g.parts();
+            WorkRef* const out = ws + ns[g.block_form];
+            for (uint32_t k = 0; k < parts; ++k) out[k] = WorkRef{i, k};
+            ns[g.block_form] += parts;
         }
         Check(hipMemcpyAsync(work_prep_.get(), wp, np * sizeof(WorkRef), hipMemcpyHostToDevice, s),
               "upload prepare work");
-        Check(hipMemcpyAsync(work_scale_.get(), ws, ns * sizeof(WorkRef), hipMemcpyHostToDevice, s),
+        Check(hipMemcpyAsync(work_scale_.get(), ws, scale_work * sizeof(WorkRef), hipMemcpyHostToDevice, s),
               "upload scale work");
         wprep = work_prep_.as<WorkRef>();
         wscale = work_scale_.as<WorkRef>();
@@ -445,12 +452,17 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
     for (uint32_t c = 0; c < chunks; ++c) {
         const uint32_t i0 = chunk_begin(c), i1 = chunk_begin(c + 1);
         if (t != s) Check(hipStreamWaitEvent(t, Ev(4 * c + 1).get(), 0), "order scale after prepare");
-        const auto ns = static_cast<uint32_t>(scale_at[i1] - scale_at[i0]);
         if (t != s) Check(hipEventRecord(Ev(4 * c + 2).get(), t), "hipEventRecord");
         const StageEnd scaled(Ev(4 * c + 3), t, record);
-        Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, uniform ? nullptr : wscale + scale_at[i0], ns,
-                          g0.parts(), g0.block_form, t, persistent, scaled.rides),
-              "launch scale");
+        const bool blocks_last = scale_at[1][i1] != scale_at[1][i0];
+        for (bool form : {false, true}) {
+            const auto ns = static_cast<uint32_t>(scale_at[form][i1] - scale_at[form][i0]);
+            if (ns == 0 && form != blocks_last) continue;
+            const WorkRef* work = uniform ? nullptr : wscale + (form ? scale_at[0][count] : 0) + scale_at[form][i0];
+            Check(LaunchScale(fmt, blur, map, uniform ? dpairs + i0 : dpairs, work, ns, g0.parts(), form, t, persistent,
+                              form == blocks_last ? scaled.rides : nullptr),
+                  "launch scale");
+        }
         scaled.Record();
     }
     const StageEnd reduced(Ev(DoneEvent()), t, record);
@@ -916,13 +928,16 @@ const vqm_ss2_batch_config& ValidatedBatch(const vqm_ss2_batch_config& config) {
 }  // namespace
 
 // A batch's default strip shape for a geometry, chosen when the geometry is
-// first submitted with `pairs` pairs of it (DefaultStripRows, RowParts).
-void Batch::SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs) {
+// first submitted with `pairs` pairs of it (DefaultStripRows, RowParts), alone
+// or with others, whose launch is long enough for the strip form.
+void Batch::SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs, bool alone) {
     const auto format = static_cast<PlaneFormat>(config_.plane_format);
     const auto cus = static_cast<uint32_t>(std::max(ctx_.cus, 1));
     const uint32_t rows = DefaultStripRows(width, height, format, config_.strip_cols, pairs, cus);
+    const bool block_form = alone && config_.strip_cols == 0 && config_.persistent == 0 &&
+                            PrefersBlocks(width, height, format, pairs, cus);
     pools_.SetStripShape(width, height, rows, config_.strip_cols,
-                         RowParts(width, height, format, rows, config_.strip_cols, pairs, cus));
+                         block_form ? 0 : RowParts(width, height, format, rows, config_.strip_cols, pairs, cus));
 }
 
 Batch::Batch(const vqm_ss2_batch_config& config)
@@ -975,7 +990,7 @@ uint64_t Batch::Submit(const vqm_ss2_device_pair* pairs, uint32_t count) {
     for (const auto& [geometry, n] : per_geometry) {
         const auto [w, h] = geometry;
         if (config_.strip_rows == 0 && !pools_.HasPlan(w, h) && !pools_.HasShape(w, h))
-            SetDefaultShape(w, h, n);
+            SetDefaultShape(w, h, n, per_geometry.size() == 1);
         pools_.PlanFor(w, h);
     }
     std::vector<Taken> taken;

@@ -409,7 +409,7 @@ public:
     // Fixes the strip shape of a geometry not used yet (a shape tuned
     // earlier, or by another process).
     void SetShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint32_t strip_cols);
-    void SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs);
+    void SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs, bool alone);
 
 private:
     struct Taken {
