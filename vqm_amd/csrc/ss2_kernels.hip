@@ -1213,8 +1213,8 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
 // from level 2 on). Rows pass through one copy of the code: 9.9 KB against
 // 25. 300 pairs: 4.07 -> 3.80 ms, of which the shorter root alone gave none
 // while the waves waited at barriers; one 4K pair 53.7 -> 45.9 us; 100 pairs
-// in the mixed form 0.90 -> 0.86 ms. A 96x64 pair, whose time is one wave's
-// chain of rows, takes 11.5 us against 9.8.
+// in the mixed form 0.90 -> 0.86 ms. (Launches of few tiles, whose time is one
+// wave's chain of rows, take the split form below.)
 //
 // Registers: 92 in the reference form, 91 in the difference form (five waves
 // a SIMD), 128 in the general decode (four).
@@ -1235,6 +1235,149 @@ prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ w
                                         src1, lds[wave]);
         if constexpr (General) __syncthreads();  // the next tile reuses the chroma window
     }
+}
+
+// The prepare kernel's split form, for launches of few tiles, whose time is one
+// wave's chain: four waves take a wave's 64 x 16 pixels, wave r the rows
+// 4 ly + r, and pass the boxes on through LDS in the same order of additions:
+// waves 1 and 3 finish the two level-1 rows, wave 3 level 2, and wave 0 levels
+// 3 and 4 meanwhile. Table-decoded images only; the same samples bit for bit.
+//
+// What bounds it: the launch, the reads of the descriptor, the plan and the row
+// (2,900 cycles of the other form's 16,700 at 96x64), and the chain of one row's
+// roots, where the other form has four rows' and three levels' (13,800). 48
+// registers. Prepare of a launch, reference form: one pair of 96x64 9.0 -> 5.1
+// us, 512x512 9.2 -> 6.3, 1080p 19.9 -> 17.2, 8 pairs of 853x479 26.0 -> 24.9.
+// The exchange and its three barriers are work of their own, so it loses where
+// the device is full anyway.
+//
+// Up to 14 tiles a CU, where the forms met: 3,360 tiles 24.9 us against 26.0,
+// 3,600 (2560x1440) 24.1 both, 6,720 40.8 against 39.2, 4K (8,160) 45.4 against
+// 41.2; U16 planes 24.5 against 24.9, 22.8 against 23.1, 37.9 against 36.3.
+constexpr uint32_t kSplitTiles = 14 * 256;
+
+template <typename Lay, bool Ref>
+__global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __restrict__ pairs,
+                                                            const WorkRef* __restrict__ work, uint32_t tiles,
+                                                            uint32_t tiles_per_image, const float* __restrict__ lut_g,
+                                                            const uint8_t* src0, const uint8_t* src1) {
+    using Fmt = typename Lay::Fmt;
+    constexpr uint32_t kHalves = kPrepTileH / kWaveRows;
+    __shared__ __align__(16) PrepareLds lds[4];  // a decode table a wave; the levels in the first
+    __shared__ float boxes1[2][2][3][64], boxes2[3][64];  // sums of the rows above
+    const uint32_t r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t entry = 4u * lane;
+    const f32x4 table = *reinterpret_cast<GlobalAS<const f32x4>*>(as_global(lut_g) + entry);
+    const uint32_t l = xcd_remap(blockIdx.x, tiles * kHalves);
+    const TileRef tr = resolve_tile(l / kHalves, pairs, work, tiles_per_image);
+    ConstAS<PairDesc>* pdp = tr.pdp;
+    ConstAS<Plan>* plan = tr.plan;
+    const uint32_t X0 = tr.X0, Y0 = tr.Y0 + kWaveRows * (l % kHalves);
+    const uint32_t W = plan->width, H = plan->height, levels = plan->levels;
+    if (Y0 >= H) return;  // the image ends above these rows
+    const uint32_t lx = lane % 16u, ly = lane / 16u;
+    GlobalAS<uint8_t>* planes =
+        as_global(static_cast<uint8_t*>(pdp->planes)) + (tr.image ? plan->image_bytes : 0);
+    const uint8_t* src_ptr = tr.image ? (src1 != nullptr ? src1 : pdp->src[1])
+                                      : (src0 != nullptr ? src0 : pdp->src[0]);
+    GlobalAS<const uint8_t>* src = as_global(src_ptr);
+    const uint32_t bx = X0 + 4u * lx, W1 = plan->w[1], H1 = plan->h[1];
+
+    // The base row, clamped as in prepare_tile.
+    const uint32_t y = Y0 + 4u * ly + r;
+    const uint32_t yc = min(min(Y0 + 4u * ly + (r & 2u), 2u * (H1 - 1u)) + (r & 1u), H - 1u);
+    const bool whole = bx + 3u < W;
+    uint32_t bytes[3] = {};  // a lane's four samples of each channel
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+        GlobalAS<const uint8_t>* row = src + c * static_cast<uint64_t>(plan->plane_stride) + static_cast<uint64_t>(yc) * W;
+        if (whole) {
+            bytes[c] = reinterpret_cast<GlobalAS<const Bytes4>*>(row + bx)->v;
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                bytes[c] |= static_cast<uint32_t>(row[min(min(bx + (j & 2u), 2u * (W1 - 1u)) + (j & 1u), W - 1u)]) << (8u * j);
+        }
+    }
+    *reinterpret_cast<f32x4*>(lds[r].lut + entry) = table;
+    wave_fence();
+    float lin[4][3];
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+        lin[0][c] = table_at<0>(lds[r].lut, bytes[c]);
+        lin[1][c] = table_at<1>(lds[r].lut, bytes[c]);
+        lin[2][c] = table_at<2>(lds[r].lut, bytes[c]);
+        lin[3][c] = table_at<3>(lds[r].lut, bytes[c]);
+    }
+    // The even rows' half of the level-1 boxes, ahead of their roots.
+    if ((r & 1u) == 0u) {
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c)
+#pragma unroll
+            for (uint32_t jj = 0; jj < 2; ++jj) boxes1[r / 2u][jj][c][lane] = (0.0f + lin[2 * jj][c]) + lin[2 * jj + 1][c];
+    }
+    __syncthreads();
+    const uint32_t gx1 = X0 / 2u + 2u * lx, gy1 = Y0 / 2u + 2u * ly + r / 2u;
+    float v1[2][3] = {}, s2[3] = {0.0f, 0.0f, 0.0f};
+    if ((r & 1u) != 0u) {
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+#pragma unroll
+            for (uint32_t jj = 0; jj < 2; ++jj) {
+                v1[jj][c] = boxes1[r / 2u][jj][c][lane] + lin[2 * jj][c];
+                v1[jj][c] = v1[jj][c] + lin[2 * jj + 1][c];
+                v1[jj][c] = linear_sample<Lay>(v1[jj][c] * 0.25f);
+            }
+            if (r == 1u) boxes2[c][lane] = (0.0f + v1[0][c]) + v1[1][c];
+        }
+    }
+    __syncthreads();
+    if (r == 3u) {
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            s2[c] = boxes2[c][lane] + v1[0][c];
+            s2[c] = s2[c] + v1[1][c];
+            s2[c] = linear_sample<Lay>(s2[c] * 0.25f);
+            lds[0].level2[c][lane] = s2[c];
+        }
+    }
+    __syncthreads();
+
+    const uint32_t mask0 = plan->mask[0], mask1 = plan->mask[1], mask2 = plan->mask[2];
+    if (mask0 != 0u && y < H) {
+        const uint64_t at = static_cast<uint64_t>(y + kPadTop) * plan->pitch[0] + bx + kPadLeft;
+        xyb_group<Ref, 4, false>(lin, mask0, [&](uint32_t c, const float (&v)[4]) {
+            auto* p = plane_at<Fmt>(planes, plan->plane_off[0][c]) + at;
+            if (whole) {
+                Fmt::store4(p, v);
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (bx + j < W) Fmt::store1(p + j, v[j]);
+            }
+        });
+    }
+    if ((r & 1u) != 0u && levels >= 2u && mask1 != 0u && gy1 < H1) {
+        const uint64_t at = static_cast<uint64_t>(gy1 + kPadTop) * plan->pitch[1] + gx1 + kPadLeft;
+        xyb_group<Ref, 2, false>(v1, mask1, [&](uint32_t c, const float (&v)[2]) {
+            auto* p = plane_at<Fmt>(planes, plan->plane_off[1][c]) + at;
+            if (gx1 + 1u < W1) {
+                Fmt::store2(p, v[0], v[1]);
+            } else if (gx1 < W1) {
+                Fmt::store1(p, v[0]);
+            }
+        });
+    }
+    const uint32_t gx2 = X0 / 4u + lx, gy2 = Y0 / 4u + ly;
+    if (r == 2u && levels >= 3u && mask2 != 0u && gx2 < plan->w[2] && gy2 < plan->h[2]) {
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) s2[c] = lds[0].level2[c][lane];
+        const uint64_t at = static_cast<uint64_t>(gy2 + kPadTop) * plan->pitch[2] + gx2 + kPadLeft;
+        xyb_group<Ref, 1, false>(&s2, mask2, [&](uint32_t c, const float (&v)[1]) {
+            Fmt::store1(plane_at<Fmt>(planes, plan->plane_off[2][c]) + at, v[0]);
+        });
+    }
+    if (r == 0u && levels >= 4u) prepare_coarse<Lay, Ref, false>(plan, planes, X0, Y0, lane, lds[0]);
 }
 
 // ---- scale ------------------------------------------------------------------
@@ -1967,6 +2110,11 @@ template <typename Lay, bool General, bool Ref>
 hipError_t launch_prepare_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t tiles,
                             const float* lut, const uint8_t* src0, const uint8_t* src1, bool persistent,
                             hipStream_t stream, hipEvent_t done) {
+    if constexpr (!General) {
+        if (!persistent && blocks <= kSplitTiles)
+            return Dispatch(&prepare_split_kernel<Lay, Ref>, blocks * (kPrepTileH / kWaveRows), 256, stream, done, pairs,
+                            work, blocks, tiles, lut, src0, src1);
+    }
     constexpr uint32_t kThreads = 64 * kPrepWaves<General>, kBlocksPerTile = kPrepTileH / kWaveRows / kPrepWaves<General>;
     const uint32_t grid = GridOf(&prepare_kernel<Lay, General, Ref>, kThreads, blocks * kBlocksPerTile, persistent);
     return Dispatch(&prepare_kernel<Lay, General, Ref>, grid, kThreads, stream, done, pairs, work, blocks, tiles, lut,
