@@ -162,13 +162,15 @@ typedef struct vqm_ss2_config {
     uint32_t strip_rows;        /* output rows per scale work item, a multiple
                                    of 8 up to 1024; 0 = chosen for the geometry
                                    as a one-pair batch's on a whole MI355X
-                                   (below): 16 rows at 1080p, 64 at 4K */
+                                   (below): 64 rows at 4K; up to 3200x1800 (with
+                                   16-bit planes 1600x900) blocks of 32 rows by
+                                   64 columns where strip_cols is 0 too */
     uint64_t input_bytes;       /* caller-owned image pool (AllocateImage), default 0 */
     uint32_t graph;             /* 1: each pair replays one HIP graph of the
-                                   descriptor upload, the three kernels and the
-                                   norm read-back, captured on first use; 0
-                                   (default): eager launches, which measured
-                                   slightly faster. No reference counterpart. */
+                                   descriptor upload and the three kernels,
+                                   captured on first use; 0 (default): eager
+                                   launches, which measured faster (a 1080p pair
+                                   72 us against 87). No reference counterpart. */
     uint32_t chroma_filter;     /* subsampled chroma upsampling: 0 bilinear
                                    (default), 1 bicubic, 2 lanczos
                                    (Ssimulacra2Config::chroma_filter) */
@@ -398,7 +400,10 @@ typedef struct vqm_ss2_batch_config {
                                 has four work items per wave slot of the
                                 device, else 128 when it has one, else 64 or
                                 32, the tallest that gives one per SIMD, else
-                                16 (servers: 64) */
+                                16 (servers: 64); a geometry first submitted
+                                alone in a launch of at most 20 blocks of 32
+                                rows by 64 columns a CU (6 with 16-bit planes)
+                                takes those */
     uint32_t max_pairs;      /* pairs per submission */
     uint32_t chunks;         /* 0 or 1: prepare, then scale, on one stream; 2..16:
                                 runs of consecutive pairs whose scale launches
@@ -420,10 +425,9 @@ typedef struct vqm_ss2_batch_config {
                                 time its shape (geometry, pair count) is seen;
                                 its stage times then report the whole graph
                                 as the prepare stage. 2: the same for
-                                submissions of up to 8 pairs, where the launch
-                                overhead shows (+16% for one 1080p pair, +6%
-                                for four, nothing from 16 on; the Python
-                                binding's default). 0: eager. */
+                                submissions of up to 8 pairs (the Python
+                                binding's default). 0: eager, 3-7% faster on
+                                one to four 1080p pairs. */
 } vqm_ss2_batch_config;
 
 /* One pair of caller-owned device images (packed u8 sRGB RGB). */
@@ -459,7 +463,7 @@ int vqm_ss2_batch_pool_bytes(const vqm_ss2_batch* batch, uint64_t* bytes);
  * its first submission, for example a shape vqm_ss2_autotune chose in an
  * earlier process; it takes precedence over `autotune`. LOGIC_ERROR once
  * the geometry has been submitted. One launch may mix strip widths (one
- * scale kernel launch per width). */
+ * scale kernel launch for both widths). */
 int vqm_ss2_batch_set_shape(vqm_ss2_batch* batch, uint32_t width, uint32_t height, uint32_t strip_rows,
                             uint32_t strip_cols);
 
