@@ -1967,6 +1967,9 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(const PairDesc* 
         if (slot & 1u) value = sqrt(sqrt(value));
     }
     const uint32_t k = slot < 2u ? 2u * c + slot : 6u + 4u * c + (slot - 2u);
+    // Coherent host memory, or the caller's on the device: seen by the host once
+    // it has waited for an event behind this kernel. (System-scope stores took
+    // 32 to 42 us for 300 pairs, these 18.)
     as_global(pdp->norms)[level * 18u + k] = value;
 }
 
