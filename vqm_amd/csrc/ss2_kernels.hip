@@ -653,11 +653,12 @@ __device__ bool chroma_window(ConstAS<SourceDesc>* d, uint32_t x_first, uint32_t
     return w->cols * w->rows <= kChromaWindow;
 }
 
-// Block-wide: thread `tid` loads every 128th entry of the window.
+// Block-wide: thread `tid` of `threads` loads every threads-th entry of the
+// window.
 __device__ void stage_chroma(ConstAS<SourceDesc>* d, GlobalAS<const uint8_t>* src, const ChromaWindow& w,
-                             uint32_t tid, float2* window) {
+                             uint32_t tid, uint32_t threads, float2* window) {
     const uint32_t n = w.cols * w.rows;
-    for (uint32_t i = tid; i < n; i += 128u) {
+    for (uint32_t i = tid; i < n; i += threads) {
         const uint32_t r = i / w.cols, c = i - r * w.cols;
         const uint32_t ix = tap_index(w.x0 + static_cast<int>(c), d->plane_w[1]);
         const uint32_t iy = tap_index(w.y0 + static_cast<int>(r), d->plane_h[1]);
@@ -1093,7 +1094,7 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
             if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0) &&
                 decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), tr.Y0,
                                       min(tr.Y0 + kPrepTileH - 1u, H - 1u), &cw)) {
-                decode::stage_chroma(sd, src, cw, threadIdx.x, chroma);
+                decode::stage_chroma(sd, src, cw, threadIdx.x, 64u * kPrepWaves<General>, chroma);
                 window = chroma;
                 __syncthreads();
             }
@@ -1267,7 +1268,8 @@ prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ w
 // wave's chain: four waves take a wave's 64 x 16 pixels, wave r the rows
 // 4 ly + r, and pass the boxes on through LDS in the same order of additions:
 // waves 1 and 3 finish the two level-1 rows, wave 3 level 2, and wave 0 levels
-// 3 and 4 meanwhile. Table-decoded images only; the same samples bit for bit.
+// 3 and 4 meanwhile. The same samples bit for bit. In the general decode the
+// block stages the chroma of its 16 rows.
 //
 // What bounds it: the launch, the reads of the descriptor, the plan and the row
 // (2,900 cycles of the other form's 16,700 at 96x64), and the chain of one row's
@@ -1280,9 +1282,12 @@ prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ w
 // Up to 14 tiles a CU, where the forms met: 3,360 tiles 24.9 us against 26.0,
 // 3,600 (2560x1440) 24.1 both, 6,720 40.8 against 39.2, 4K (8,160) 45.4 against
 // 41.2; U16 planes 24.5 against 24.9, 22.8 against 23.1, 37.9 against 36.3.
-constexpr uint32_t kSplitTiles = 14 * 256;
+// General decode, up to 4 tiles a CU: 512x512 8-bit 4:2:0 20.2 -> 10.9 us, 10-bit
+// PQ 23.3 -> 11.8, 1280x720 (920 tiles) 24.9 -> 21.0 and 31.6 -> 24.4; 1080p
+// (2,040) 33.7 against 36.6 and 42.0 against 41.2. 86 registers.
+template <bool General> constexpr uint32_t kSplitTiles = (General ? 4 : 14) * 256;
 
-template <typename Lay, bool Ref>
+template <typename Lay, bool General, bool Ref>
 __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __restrict__ pairs,
                                                             const WorkRef* __restrict__ work, uint32_t tiles,
                                                             uint32_t tiles_per_image, const float* __restrict__ lut_g,
@@ -1309,31 +1314,55 @@ __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __re
     GlobalAS<const uint8_t>* src = as_global(src_ptr);
     const uint32_t bx = X0 + 4u * lx, W1 = plan->w[1], H1 = plan->h[1];
 
-    // The base row, clamped as in prepare_tile.
+    // The base row and columns, clamped as in prepare_tile.
     const uint32_t y = Y0 + 4u * ly + r;
     const uint32_t yc = min(min(Y0 + 4u * ly + (r & 2u), 2u * (H1 - 1u)) + (r & 1u), H - 1u);
+    auto base_col = [&](uint32_t j) -> uint32_t { return min(min(bx + (j & 2u), 2u * (W1 - 1u)) + (j & 1u), W - 1u); };
     const bool whole = bx + 3u < W;
-    uint32_t bytes[3] = {};  // a lane's four samples of each channel
-#pragma unroll
-    for (uint32_t c = 0; c < 3; ++c) {
-        GlobalAS<const uint8_t>* row = src + c * static_cast<uint64_t>(plan->plane_stride) + static_cast<uint64_t>(yc) * W;
-        if (whole) {
-            bytes[c] = reinterpret_cast<GlobalAS<const Bytes4>*>(row + bx)->v;
-        } else {
-#pragma unroll
-            for (uint32_t j = 0; j < 4; ++j)
-                bytes[c] |= static_cast<uint32_t>(row[min(min(bx + (j & 2u), 2u * (W1 - 1u)) + (j & 1u), W - 1u)]) << (8u * j);
+    float lin[4][3];
+    bool from_table = true;
+    if constexpr (General) {
+        const SourceDesc* sdp = tr.image ? pdp->source[1] : pdp->source[0];
+        if (sdp != nullptr && as_const(sdp)->kind != 0u) {
+            from_table = false;
+            ConstAS<SourceDesc>* sd = as_const(sdp);
+            __shared__ float2 chroma[decode::kChromaWindow];
+            const float2* window = nullptr;
+            decode::ChromaWindow cw{0, 0, 0, 0};
+            if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0) &&
+                decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), Y0, min(Y0 + kWaveRows - 1u, H - 1u), &cw)) {
+                decode::stage_chroma(sd, src, cw, threadIdx.x, 256u, chroma);
+                window = chroma;
+                __syncthreads();
+            }
+            const uint32_t col[4] = {base_col(0), base_col(1), base_col(2), base_col(3)};
+            decode::BilinearColumns columns{};
+            if (window != nullptr && sd->filter == 0) columns = decode::bilinear_columns(sd, cw, col);
+            decode::row4(sd, src, window, cw, columns, bx, col, yc, W, lin);
         }
     }
-    *reinterpret_cast<f32x4*>(lds[r].lut + entry) = table;
-    wave_fence();
-    float lin[4][3];
+    if (from_table) {
+        uint32_t bytes[3] = {};  // a lane's four samples of each channel
 #pragma unroll
-    for (uint32_t c = 0; c < 3; ++c) {
-        lin[0][c] = table_at<0>(lds[r].lut, bytes[c]);
-        lin[1][c] = table_at<1>(lds[r].lut, bytes[c]);
-        lin[2][c] = table_at<2>(lds[r].lut, bytes[c]);
-        lin[3][c] = table_at<3>(lds[r].lut, bytes[c]);
+        for (uint32_t c = 0; c < 3; ++c) {
+            GlobalAS<const uint8_t>* row =
+                src + c * static_cast<uint64_t>(plan->plane_stride) + static_cast<uint64_t>(yc) * W;
+            if (whole) {
+                bytes[c] = reinterpret_cast<GlobalAS<const Bytes4>*>(row + bx)->v;
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) bytes[c] |= static_cast<uint32_t>(row[base_col(j)]) << (8u * j);
+            }
+        }
+        *reinterpret_cast<f32x4*>(lds[r].lut + entry) = table;
+        wave_fence();
+#pragma unroll
+        for (uint32_t c = 0; c < 3; ++c) {
+            lin[0][c] = table_at<0>(lds[r].lut, bytes[c]);
+            lin[1][c] = table_at<1>(lds[r].lut, bytes[c]);
+            lin[2][c] = table_at<2>(lds[r].lut, bytes[c]);
+            lin[3][c] = table_at<3>(lds[r].lut, bytes[c]);
+        }
     }
     // The even rows' half of the level-1 boxes, ahead of their roots.
     if ((r & 1u) == 0u) {
@@ -1372,7 +1401,7 @@ __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __re
     const uint32_t mask0 = plan->mask[0], mask1 = plan->mask[1], mask2 = plan->mask[2];
     if (mask0 != 0u && y < H) {
         const uint64_t at = static_cast<uint64_t>(y + kPadTop) * plan->pitch[0] + bx + kPadLeft;
-        xyb_group<Ref, 4, false>(lin, mask0, [&](uint32_t c, const float (&v)[4]) {
+        xyb_group<Ref, 4, General>(lin, mask0, [&](uint32_t c, const float (&v)[4]) {
             auto* p = plane_at<Fmt>(planes, plan->plane_off[0][c]) + at;
             if (whole) {
                 Fmt::store4(p, v);
@@ -1385,7 +1414,7 @@ __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __re
     }
     if ((r & 1u) != 0u && levels >= 2u && mask1 != 0u && gy1 < H1) {
         const uint64_t at = static_cast<uint64_t>(gy1 + kPadTop) * plan->pitch[1] + gx1 + kPadLeft;
-        xyb_group<Ref, 2, false>(v1, mask1, [&](uint32_t c, const float (&v)[2]) {
+        xyb_group<Ref, 2, General>(v1, mask1, [&](uint32_t c, const float (&v)[2]) {
             auto* p = plane_at<Fmt>(planes, plan->plane_off[1][c]) + at;
             if (gx1 + 1u < W1) {
                 Fmt::store2(p, v[0], v[1]);
@@ -1399,11 +1428,11 @@ __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __re
 #pragma unroll
         for (uint32_t c = 0; c < 3; ++c) s2[c] = lds[0].level2[c][lane];
         const uint64_t at = static_cast<uint64_t>(gy2 + kPadTop) * plan->pitch[2] + gx2 + kPadLeft;
-        xyb_group<Ref, 1, false>(&s2, mask2, [&](uint32_t c, const float (&v)[1]) {
+        xyb_group<Ref, 1, General>(&s2, mask2, [&](uint32_t c, const float (&v)[1]) {
             Fmt::store1(plane_at<Fmt>(planes, plan->plane_off[2][c]) + at, v[0]);
         });
     }
-    if (r == 0u && levels >= 4u) prepare_coarse<Lay, Ref, false>(plan, planes, X0, Y0, lane, lds[0]);
+    if (r == 0u && levels >= 4u) prepare_coarse<Lay, Ref, General>(plan, planes, X0, Y0, lane, lds[0]);
 }
 
 // ---- scale ------------------------------------------------------------------
@@ -2139,11 +2168,9 @@ template <typename Lay, bool General, bool Ref>
 hipError_t launch_prepare_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t tiles,
                             const float* lut, const uint8_t* src0, const uint8_t* src1, bool persistent,
                             hipStream_t stream, hipEvent_t done) {
-    if constexpr (!General) {
-        if (!persistent && blocks <= kSplitTiles)
-            return Dispatch(&prepare_split_kernel<Lay, Ref>, blocks * (kPrepTileH / kWaveRows), 256, stream, done, pairs,
-                            work, blocks, tiles, lut, src0, src1);
-    }
+    if (!persistent && blocks <= kSplitTiles<General>)
+        return Dispatch(&prepare_split_kernel<Lay, General, Ref>, blocks * (kPrepTileH / kWaveRows), 256, stream, done,
+                        pairs, work, blocks, tiles, lut, src0, src1);
     constexpr uint32_t kThreads = 64 * kPrepWaves<General>, kBlocksPerTile = kPrepTileH / kWaveRows / kPrepWaves<General>;
     const uint32_t grid = GridOf(&prepare_kernel<Lay, General, Ref>, kThreads, blocks * kBlocksPerTile, persistent);
     return Dispatch(&prepare_kernel<Lay, General, Ref>, grid, kThreads, stream, done, pairs, work, blocks, tiles, lut,
