@@ -382,6 +382,31 @@ WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan) {
     return l;
 }
 
+NoAllocPlan PlanNoAlloc(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
+                        uint32_t strip_cols) {
+    const uint32_t rows = SinglePairStripRows(width, height, format, strip_rows, strip_cols);
+    const uint32_t row_parts = SinglePairRowParts(width, height, format, strip_rows, strip_cols);
+    auto partials_at = [](const Plan& p) {
+        return Align(kNoAllocItemsAt + static_cast<uint64_t>(p.items) * sizeof(ScaleItem), 256);
+    };
+    auto planes_at = [&](const Plan& p, uint64_t sums) { return Align(partials_at(p) + sums * 6 * sizeof(double), 256); };
+    const Plan strips = FillPlan(width, height, format, rows, strip_cols);
+    const uint64_t need = planes_at(strips, strips.items) + 2 * strips.image_bytes;
+    if (need > kNoAllocPairBytes)
+        Fail(VQM_INVALID_ARGUMENT,
+             "a " + std::to_string(width) + "x" + std::to_string(height) + " pair in this plane format needs " +
+                 std::to_string(need) + " bytes of scratch; the allocation-free entry point takes pairs of up to " +
+                 std::to_string(kNoAllocPairBytes) + " (use a pipeline for larger pairs)");
+    NoAllocPlan n;
+    n.plan = FillPlan(width, height, format, rows, strip_cols, row_parts);
+    n.block_form = row_parts == 0;
+    n.parts = static_cast<uint64_t>(n.plan.items) << n.plan.part_shift;
+    n.partials_at = partials_at(n.plan);
+    n.planes_at = planes_at(n.plan, n.parts);
+    if (n.planes_at + 2 * n.plan.image_bytes > kNoAllocScratchBytes) Fail(VQM_RUNTIME_ERROR, "the scratch is too small");
+    return n;
+}
+
 uint64_t AlgorithmicBytes(const GeometryPlan& plan) {
     const Plan& p = plan.plan;
     uint64_t bytes = 0;  // stored plane bytes of one image, unpadded

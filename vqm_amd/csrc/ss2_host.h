@@ -137,6 +137,28 @@ struct WorkspaceLayout {
 };
 WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan);
 
+// The allocation-free entry point's pairs. It takes a pair whose regions of
+// fixed size, items, one partial sum a strip and planes of both images fit
+// kNoAllocPairBytes, whichever form of the scale kernel runs. Its scratch is
+// larger: a strip has up to eight parts, of 48 bytes each, and the planes
+// under a part (8 rows or more by 64 columns, two images of two bytes a sample
+// or more) hold 2,048 bytes or more, so the parts of such a pair take at most
+// 48 / 2048 of kNoAllocPairBytes, 3 MiB.
+inline constexpr uint64_t kNoAllocPairBytes = 128ull << 20;
+inline constexpr uint64_t kNoAllocScratchBytes = 132ull << 20;
+inline constexpr uint64_t kNoAllocItemsAt = 2048;  // behind the regions of fixed size
+struct NoAllocPlan {
+    Plan plan{};
+    bool block_form = false;
+    uint64_t parts = 0;                       // scale blocks
+    uint64_t partials_at = 0, planes_at = 0;  // scratch offsets
+};
+// The plan of a single-pair pipeline of this geometry, so that both give the
+// same sums. Throws Error{VQM_INVALID_ARGUMENT} for a pair that it does not
+// take.
+NoAllocPlan PlanNoAlloc(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
+                        uint32_t strip_cols);
+
 // Offset bookkeeping of a device arena: ranges of a fixed capacity handed
 // out in 256-byte multiples by first fit over an address-ordered free list,
 // neighbours merged on release.

@@ -34,7 +34,6 @@ namespace {
 constexpr uint64_t kPairAt = 0;
 constexpr uint64_t kPlanAt = 256;
 constexpr uint64_t kLutAt = 1024;
-constexpr uint64_t kItemsAt = 2048;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
@@ -43,8 +42,6 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 // looked up once with that device current.
 std::mutex g_mutex;
 void* g_scratch[kMaxDevices] = {};
-
-uint64_t Align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
 // Everything the setup kernel writes, passed by value.
 struct SetupArgs {
@@ -80,7 +77,7 @@ __global__ __launch_bounds__(256) void setup_kernel(SetupArgs args, uint8_t* bas
 
 static_assert(sizeof(PairDesc) <= kPlanAt - kPairAt, "pair descriptor region");
 static_assert(sizeof(Plan) <= kLutAt - kPlanAt, "plan region");
-static_assert(256 * sizeof(float) <= kItemsAt - kLutAt, "decode table region");
+static_assert(256 * sizeof(float) <= kNoAllocItemsAt - kLutAt, "decode table region");
 
 // The calling thread's current device's scratch address.
 uint8_t* DeviceScratch() {
@@ -121,27 +118,10 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
              "the allocation-free entry point takes 8-bit full-range sRGB RGB images only "
              "(score other formats through a pipeline)");
 
-    // The strip height a pipeline of this geometry takes, so both give the
-    // same sums.
     SetupArgs args{};
-    const uint32_t row_parts =
-        SinglePairRowParts(config.width, config.height, format, config.strip_rows, config.strip_cols);
-    args.plan = FillPlan(config.width, config.height, format,
-                         SinglePairStripRows(config.width, config.height, format, config.strip_rows,
-                                             config.strip_cols),
-                         config.strip_cols,
-                         row_parts);
+    const NoAllocPlan n = PlanNoAlloc(config.width, config.height, format, config.strip_rows, config.strip_cols);
+    args.plan = n.plan;
     const Plan& p = args.plan;
-    const uint64_t parts = static_cast<uint64_t>(p.items) << p.part_shift;
-    const uint64_t partials_at = Align256(kItemsAt + static_cast<uint64_t>(p.items) * sizeof(ScaleItem));
-    const uint64_t planes_at = Align256(partials_at + parts * 6 * sizeof(double));
-    const uint64_t need = planes_at + 2 * p.image_bytes;
-    if (need > kNoAllocScratchBytes)
-        Fail(VQM_INVALID_ARGUMENT,
-             "a " + std::to_string(config.width) + "x" + std::to_string(config.height) +
-                 " pair in this plane format needs " + std::to_string(need) +
-                 " bytes of scratch; the allocation-free entry point holds " +
-                 std::to_string(kNoAllocScratchBytes) + " (use a pipeline for larger pairs)");
 
     uint8_t* base = DeviceScratch();
     const std::array<float, 256> lut = SrgbTable();
@@ -149,24 +129,24 @@ uint32_t ScoreDeviceNoAlloc(const vqm_ss2_config& config, const vqm_device_image
     PairDesc& pd = args.pair;
     pd.src[0] = static_cast<const uint8_t*>(a.data);
     pd.src[1] = static_cast<const uint8_t*>(b.data);
-    pd.planes = base + planes_at;
-    pd.partials = reinterpret_cast<double*>(base + partials_at);
+    pd.planes = base + n.planes_at;
+    pd.partials = reinterpret_cast<double*>(base + n.partials_at);
     pd.norms = norms;
     pd.plan = reinterpret_cast<const Plan*>(base + kPlanAt);
-    pd.items = reinterpret_cast<const ScaleItem*>(base + kItemsAt);
+    pd.items = reinterpret_cast<const ScaleItem*>(base + kNoAllocItemsAt);
 
     const uint64_t plane_words = 2 * p.image_bytes / 16;  // image_bytes is a multiple of 256
     const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(plane_words / 256, 1), 2048));
-    hipLaunchKernelGGL(setup_kernel, dim3(blocks), dim3(256), 0, stream, args, base, kItemsAt, planes_at,
-                       plane_words);
+    hipLaunchKernelGGL(setup_kernel, dim3(blocks), dim3(256), 0, stream, args, base, kNoAllocItemsAt,
+                       n.planes_at, plane_words);
     Check(hipGetLastError(), "launch setup");
     const PairDesc* dpair = reinterpret_cast<const PairDesc*>(base + kPairAt);
     const float* dlut = reinterpret_cast<const float*>(base + kLutAt);
     const uint32_t tiles = p.prep_tiles_x * p.prep_tiles_y;
     Check(LaunchPrepare(format, map, false, dpair, nullptr, 2 * tiles, tiles, dlut, nullptr, nullptr, stream),
           "launch prepare");
-    Check(LaunchScale(format, config.blur, map, dpair, nullptr, static_cast<uint32_t>(parts), static_cast<uint32_t>(parts),
-                      row_parts == 0, stream),
+    const uint32_t parts = static_cast<uint32_t>(n.parts);
+    Check(LaunchScale(format, config.blur, map, dpair, nullptr, parts, parts, n.block_form, stream),
           "launch scale");
     Check(LaunchReduce(dpair, 1, stream), "launch reduce");
     return p.levels;
