@@ -409,7 +409,9 @@ typedef struct vqm_ss2_batch_config {
     uint32_t chunks;         /* 0 or 1: prepare, then scale, on one stream; 2..16:
                                 runs of consecutive pairs whose scale launches
                                 (second stream) overlap the next run's prepare */
-    uint64_t hbm_budget;     /* device bytes the workspace pool may hold, 0 = unlimited */
+    uint64_t hbm_budget;     /* device bytes the workspace pool may hold, 0 = unlimited
+                                (the pairs' planes; their descriptors, work lists
+                                and partial sums are apart from it) */
     uint32_t autotune;       /* 1: strip_rows, strip_cols and chunks come from
                                 vqm_ss2_autotune for each geometry the first
                                 time it is seen */

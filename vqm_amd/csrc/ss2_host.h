@@ -137,6 +137,12 @@ struct WorkspaceLayout {
 };
 WorkspaceLayout LayoutWorkspace(const GeometryPlan& plan);
 
+// What a pair's workspace holds in the pools of batches and servers: its
+// planes. The partials of the pairs in flight are their lane's (a strip's
+// parts have up to eight times the sums of a strip, so that workspaces with
+// them would not fit a budget that held them with one sum a strip).
+inline WorkspaceLayout PooledWorkspace(const WorkspaceLayout& layout) { return {layout.planes, 0, layout.planes}; }
+
 // The allocation-free entry point's pairs. It takes a pair whose regions of
 // fixed size, items, one partial sum a strip and planes of both images fit
 // kNoAllocPairBytes, whichever form of the scale kernel runs. Its scratch is

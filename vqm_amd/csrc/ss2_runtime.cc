@@ -184,7 +184,7 @@ Workspace::Workspace(const WorkspaceLayout& layout, uint64_t input_image_bytes, 
     // for it, so finish it before any kernel can touch the planes.
     Check(hipStreamSynchronize(nullptr), "clear workspace");
     planes = base;
-    partials = reinterpret_cast<double*>(base + layout.planes);
+    if (layout.partials > 0) partials = reinterpret_cast<double*>(base + layout.planes);
     if (input_image_bytes > 0) inputs = base + layout.total;
 }
 
@@ -217,9 +217,7 @@ const DevicePlan& WorkspacePools::PlanFor(uint32_t width, uint32_t height) {
 
 uint64_t WorkspacePools::Need(uint32_t width, uint32_t height, bool inputs) {
     const DevicePlan& plan = PlanFor(width, height);
-    uint64_t need = plan.layout.total;
-    if (inputs) need += InputArea(RequiredBytes(Srgb8Format(), width, height));
-    return need;
+    return Workspace::Bytes(PooledWorkspace(plan.layout), inputs ? RequiredBytes(Srgb8Format(), width, height) : 0);
 }
 
 std::unique_ptr<Workspace> WorkspacePools::Acquire(uint32_t width, uint32_t height, bool inputs) {
@@ -231,7 +229,8 @@ std::unique_ptr<Workspace> WorkspacePools::Acquire(uint32_t width, uint32_t heig
     }
     const DevicePlan& plan = PlanFor(width, height);
     const uint64_t input_bytes = inputs ? RequiredBytes(Srgb8Format(), width, height) : 0;
-    const uint64_t need = Workspace::Bytes(plan.layout, input_bytes);
+    const WorkspaceLayout layout = PooledWorkspace(plan.layout);
+    const uint64_t need = Workspace::Bytes(layout, input_bytes);
     void* memory = nullptr;
     if (budget_ != 0) {
         if (need > budget_) return nullptr;
@@ -251,7 +250,7 @@ std::unique_ptr<Workspace> WorkspacePools::Acquire(uint32_t width, uint32_t heig
     }
     std::unique_ptr<Workspace> ws;
     try {
-        ws = std::make_unique<Workspace>(plan.layout, input_bytes, memory);
+        ws = std::make_unique<Workspace>(layout, input_bytes, memory);
     } catch (...) {
         if (memory) arena_->Free(memory, need);
         throw;
@@ -345,13 +344,18 @@ void Lane::Launch(PlaneFormat fmt, MapForm map, const float* lut, const LaunchEn
     // form, behind all the others'.
     std::vector<uint64_t> prep_at(count + 1, 0), scale_at[2];
     for (auto& at : scale_at) at.assign(count + 1, 0);
+    uint64_t partials = 0;
+    for (uint32_t i = 0; i < count; ++i) partials += entries[i].plan->layout.partials;
+    if (partials_.bytes() < partials) partials_ = DeviceBuffer(std::max(partials, 2 * partials_.bytes()));
+    partials = 0;
     for (uint32_t i = 0; i < count; ++i) {
         const LaunchEntry& e = entries[i];
         PairDesc& pd = hp[i];
         for (int k = 0; k < 2; ++k)
             pd.src[k] = e.host[k] ? e.ws->inputs + k * ((e.image_bytes + 255) / 256 * 256) : e.src[k];
         pd.planes = e.ws->planes;
-        pd.partials = e.ws->partials;
+        pd.partials = reinterpret_cast<double*>(partials_.as<uint8_t>() + partials);
+        partials += e.plan->layout.partials;
         pd.norms = h_norms_.as<double>() + static_cast<uint64_t>(i) * kNorms;
         pd.plan = e.plan->plan.as<Plan>();
         pd.items = e.plan->items.as<ScaleItem>();

@@ -123,8 +123,9 @@ struct DevicePlan {
                uint32_t row_parts = 1);
 };
 
-// One pair's device workspace: planes (zero borders), partials and,
-// for pairs whose inputs arrive from the host, room for both input images.
+// One pair's device workspace: planes (zero borders), partials (a pipeline's;
+// PooledWorkspace has none) and, for pairs whose inputs arrive from the host,
+// room for both input images.
 // It owns its memory, or uses `bytes` at `memory` carved from an arena.
 struct Workspace {
     DeviceBuffer owned;
@@ -280,6 +281,7 @@ public:
 private:
     uint32_t max_pairs_;
     DeviceBuffer pairs_, work_prep_, work_scale_;
+    DeviceBuffer partials_;  // of the pairs of a launch; grows on demand
     PinnedBuffer h_pairs_, h_work_prep_, h_work_scale_, h_norms_;
     Stream stream_, scale_stream_;
     // Per chunk: prepare start/end, scale start (on its own stream; unused
