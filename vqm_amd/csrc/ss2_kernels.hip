@@ -41,6 +41,7 @@
 #include "ss2_cbrt.h"
 #include "ss2_common.h"
 #include "ss2_kernels.h"
+#include "ss2_launch.h"
 
 #pragma clang fp contract(off)
 
@@ -2129,21 +2130,22 @@ __global__ __launch_bounds__(256) void div_check_kernel(uint32_t mb_first, uint3
 // compute unit x compute units, rounded down to a multiple of 8 (at least
 // 8). A persistent launch uses min(work items, this) blocks, each looping
 // over its share; 0 when the runtime cannot say.
-uint32_t ResidentGrid(const void* kernel, int block_threads) {
-    int per_cu = 0, device = 0;
+uint32_t ResidentGrid(const void* kernel, int device, int block_threads) {
+    int per_cu = 0;
     hipDeviceProp_t prop{};
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block_threads, 0) != hipSuccess ||
-        hipGetDevice(&device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
-        per_cu <= 0 || prop.multiProcessorCount <= 0)
+        hipGetDeviceProperties(&prop, device) != hipSuccess || per_cu <= 0 || prop.multiProcessorCount <= 0)
         return 0;
     const uint64_t resident = static_cast<uint64_t>(per_cu) * static_cast<uint64_t>(prop.multiProcessorCount);
     return static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(8, resident / 8 * 8), 0x7FFFFFF8u));
 }
 
-template <typename K>
-uint32_t GridOf(K kernel, int block_threads, uint32_t blocks, bool persistent) {
-    if (!persistent) return blocks;
-    static const uint32_t resident = ResidentGrid(reinterpret_cast<const void*>(kernel), block_threads);
+template <auto Kernel>
+uint32_t GridOf(int block_threads, uint32_t blocks, bool persistent) {
+    int device = 0;
+    if (!persistent || hipGetDevice(&device) != hipSuccess) return blocks;
+    const uint32_t resident = OncePerKernel<Kernel>(
+        device, [&] { return ResidentGrid(reinterpret_cast<const void*>(Kernel), device, block_threads); });
     return resident == 0 ? blocks : std::min(blocks, resident);
 }
 
@@ -2172,7 +2174,7 @@ hipError_t launch_prepare_g(const PairDesc* pairs, const WorkRef* work, uint32_t
         return Dispatch(&prepare_split_kernel<Lay, General, Ref>, blocks * (kPrepTileH / kWaveRows), 256, stream, done,
                         pairs, work, blocks, tiles, lut, src0, src1);
     constexpr uint32_t kThreads = 64 * kPrepWaves<General>, kBlocksPerTile = kPrepTileH / kWaveRows / kPrepWaves<General>;
-    const uint32_t grid = GridOf(&prepare_kernel<Lay, General, Ref>, kThreads, blocks * kBlocksPerTile, persistent);
+    const uint32_t grid = GridOf<&prepare_kernel<Lay, General, Ref>>(kThreads, blocks * kBlocksPerTile, persistent);
     return Dispatch(&prepare_kernel<Lay, General, Ref>, grid, kThreads, stream, done, pairs, work, blocks, tiles, lut,
                     src0, src1);
 }
@@ -2199,7 +2201,7 @@ hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t b
     if (block_form)
         return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, blocks, 64 * kBlockWaves, stream, done, pairs, work,
                         blocks, parts);
-    const uint32_t grid = GridOf(&scale_kernel<Lay, TapsT, Ref>, 64, blocks, persistent);
+    const uint32_t grid = GridOf<&scale_kernel<Lay, TapsT, Ref>>(64, blocks, persistent);
     return Dispatch(&scale_kernel<Lay, TapsT, Ref>, grid, 64, stream, done, pairs, work, blocks, parts);
 }
 
