@@ -2140,8 +2140,11 @@ uint32_t ResidentGrid(const void* kernel, int device, int block_threads) {
     return static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(8, resident / 8 * 8), 0x7FFFFFF8u));
 }
 
+// The grid of a kernel whose blocks stride over `blocks`: all that a launch may
+// have, or the resident ones.
 template <auto Kernel>
 uint32_t GridOf(int block_threads, uint32_t blocks, bool persistent) {
+    blocks = std::min(blocks, MaxBlocks(static_cast<uint32_t>(block_threads)));
     int device = 0;
     if (!persistent || hipGetDevice(&device) != hipSuccess) return blocks;
     const uint32_t resident = OncePerKernel<Kernel>(
@@ -2198,9 +2201,16 @@ hipError_t launch_prepare_t(MapForm map, bool general, const PairDesc* pairs, co
 template <typename Lay, typename TapsT, bool Ref>
 hipError_t launch_scale_g(const PairDesc* pairs, const WorkRef* work, uint32_t blocks, uint32_t parts,
                           bool block_form, bool persistent, hipStream_t stream, hipEvent_t done) {
-    if (block_form)
-        return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, blocks, 64 * kBlockWaves, stream, done, pairs, work,
-                        blocks, parts);
+    if (block_form) {
+        // Runs of whole pairs, or of the work list.
+        constexpr uint32_t kMost = MaxBlocks(64 * kBlockWaves);
+        const uint32_t unit = work != nullptr ? 1u : parts;
+        return InRuns(blocks / unit, std::max(kMost / unit, 1u), [&](uint32_t first, uint32_t n, bool last) {
+            return Dispatch(&scale_block_kernel<Lay, TapsT, Ref>, n * unit, 64 * kBlockWaves, stream,
+                            last ? done : nullptr, work != nullptr ? pairs : pairs + first,
+                            work != nullptr ? work + first : nullptr, n * unit, parts);
+        });
+    }
     const uint32_t grid = GridOf<&scale_kernel<Lay, TapsT, Ref>>(64, blocks, persistent);
     return Dispatch(&scale_kernel<Lay, TapsT, Ref>, grid, 64, stream, done, pairs, work, blocks, parts);
 }
@@ -2292,7 +2302,9 @@ hipError_t LaunchScale(PlaneFormat format, uint32_t blur, MapForm map, const Pai
 
 hipError_t LaunchReduce(const PairDesc* pairs, uint32_t pairs_count, hipStream_t stream, hipEvent_t done) {
     if (pairs_count == 0) return Nothing(stream, done);
-    return Dispatch(&reduce_kernel, pairs_count * kRanges, kReduceThreads, stream, done, pairs);
+    return InRuns(pairs_count, MaxBlocks(kReduceThreads) / kRanges, [&](uint32_t first, uint32_t n, bool last) {
+        return Dispatch(&reduce_kernel, n * kRanges, kReduceThreads, stream, last ? done : nullptr, pairs + first);
+    });
 }
 
 }  // namespace vqm::ss2
