@@ -414,7 +414,8 @@ typedef struct vqm_ss2_batch_config {
                                 and partial sums are apart from it) */
     uint32_t autotune;       /* 1: strip_rows, strip_cols and chunks come from
                                 vqm_ss2_autotune for each geometry the first
-                                time it is seen */
+                                time it is seen, or the geometry takes the
+                                default shape above where that measured faster */
     uint32_t blur;           /* VQM_BLUR_SAMPLED or VQM_BLUR_RECURSIVE */
     uint32_t persistent;     /* 1: each kernel launches only the blocks that stay
                                 resident at once (occupancy x compute units), each
@@ -485,7 +486,10 @@ typedef struct vqm_ss2_tune_result {
 /* Times every (strip height 16/32/64/128/192/256) x (strip width 64/128) x
  * (chunks 1/2/4/8) shape for a launch of `pairs` pairs of this geometry and
  * format (rounded up to a power of two, at most 512) on the device and
- * returns the fastest; the choice is cached for the process. Shapes change
+ * returns the fastest; the choice is cached for the process. (A batch with
+ * `autotune` also times what set_shape cannot name, blocks and strips cut into
+ * bands, as a launch of no set shape takes them, and keeps to the fastest of
+ * all.) Shapes change
  * only the order in which the FP64 partial sums of the strips are added
  * (every pixel's map value and every FP32 block sum is the same), so results
  * agree to about 1e-15 relative.

@@ -347,6 +347,23 @@ bool PrefersBlocks(uint32_t width, uint32_t height, PlaneFormat format, uint64_t
     return FillPlan(width, height, format, 0, 0, 0).items * pairs <= most;
 }
 
+ScaleShape DefaultShape(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_cols, uint64_t pairs,
+                        uint32_t cus, bool blocks) {
+    const uint32_t rows = DefaultStripRows(width, height, format, strip_cols, pairs, cus);
+    if (blocks && PrefersBlocks(width, height, format, pairs, cus)) return {rows, strip_cols, 0};
+    return {rows, strip_cols, RowParts(width, height, format, rows, strip_cols, pairs, cus)};
+}
+
+std::vector<ScaleShape> TuneShapes(uint32_t width, uint32_t height, PlaneFormat format, uint64_t pairs, uint32_t cus) {
+    std::vector<ScaleShape> shapes;
+    for (uint32_t rows : kTuneRows)
+        for (uint32_t cols : kTuneCols) shapes.push_back({rows, cols, 1});
+    const ScaleShape strips = DefaultShape(width, height, format, 0, pairs, cus, false);
+    if (strips.row_parts != 1) shapes.push_back(strips);
+    shapes.push_back({strips.rows, strips.cols, 0});
+    return shapes;
+}
+
 uint32_t SinglePairRowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_rows,
                             uint32_t strip_cols) {
     if (strip_rows == 0 && strip_cols == 0 && PrefersBlocks(width, height, format, 1, kWholeDeviceCUs)) return 0;

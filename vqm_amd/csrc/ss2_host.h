@@ -6,6 +6,7 @@
 #include <array>
 #include <cstddef>
 #include <cstdint>
+#include <iterator>
 #include <map>
 #include <string>
 #include <vector>
@@ -123,6 +124,27 @@ uint32_t RowParts(uint32_t width, uint32_t height, PlaneFormat format, uint32_t 
 // Whether a scale launch of `pairs` pairs of this geometry alone takes the
 // block form.
 bool PrefersBlocks(uint32_t width, uint32_t height, PlaneFormat format, uint64_t pairs, uint32_t cus);
+
+// A scale launch's shape: FillPlan's strip_rows, strip_cols (0: the default
+// width) and row_parts.
+struct ScaleShape {
+    uint32_t rows = 64, cols = 0, row_parts = 1;
+    bool operator==(const ScaleShape&) const = default;
+};
+
+// The shape that a launch of `pairs` pairs of this geometry takes where none is
+// set: DefaultStripRows cut by RowParts, or the block form where PrefersBlocks
+// and `blocks` (the geometry alone, one block a part, no strip width set).
+ScaleShape DefaultShape(uint32_t width, uint32_t height, PlaneFormat format, uint32_t strip_cols, uint64_t pairs,
+                        uint32_t cus, bool blocks);
+
+// The shapes the autotuner times: first those that a caller can set, every
+// height of kTuneRows in both widths, then the default shape of such a launch
+// where it is another (cut strips) and the block form.
+inline constexpr uint32_t kTuneRows[] = {16, 32, 64, 128, 192, 256};
+inline constexpr uint32_t kTuneCols[] = {64, 128};
+inline constexpr size_t kTuneSettable = std::size(kTuneRows) * std::size(kTuneCols);
+std::vector<ScaleShape> TuneShapes(uint32_t width, uint32_t height, PlaneFormat format, uint64_t pairs, uint32_t cus);
 
 // RowParts of a single-pair pipeline's default height (of the geometry
 // alone, as SinglePairStripRows), or 0 for the block form, where neither

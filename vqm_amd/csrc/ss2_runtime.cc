@@ -935,13 +935,10 @@ const vqm_ss2_batch_config& ValidatedBatch(const vqm_ss2_batch_config& config) {
 // first submitted with `pairs` pairs of it (DefaultStripRows, RowParts), alone
 // or with others, whose launch is long enough for the strip form.
 void Batch::SetDefaultShape(uint32_t width, uint32_t height, uint32_t pairs, bool alone) {
-    const auto format = static_cast<PlaneFormat>(config_.plane_format);
-    const auto cus = static_cast<uint32_t>(std::max(ctx_.cus, 1));
-    const uint32_t rows = DefaultStripRows(width, height, format, config_.strip_cols, pairs, cus);
-    const bool block_form = alone && config_.strip_cols == 0 && config_.persistent == 0 &&
-                            PrefersBlocks(width, height, format, pairs, cus);
-    pools_.SetStripShape(width, height, rows, config_.strip_cols,
-                         block_form ? 0 : RowParts(width, height, format, rows, config_.strip_cols, pairs, cus));
+    pools_.SetStripShape(width, height,
+                         DefaultShape(width, height, static_cast<PlaneFormat>(config_.plane_format),
+                                      config_.strip_cols, pairs, static_cast<uint32_t>(std::max(ctx_.cus, 1)),
+                                      alone && config_.strip_cols == 0 && config_.persistent == 0));
 }
 
 Batch::Batch(const vqm_ss2_batch_config& config)
@@ -959,8 +956,8 @@ void Batch::SetShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint3
     if (pools_.HasPlan(width, height))
         Fail(VQM_LOGIC_ERROR, "the strip shape of a geometry already used cannot change");
     pools_.SetStripShape(width, height,
-                         strip_rows != 0 ? strip_rows : (config_.strip_rows != 0 ? config_.strip_rows : 128),
-                         strip_cols != 0 ? strip_cols : config_.strip_cols);
+                         {strip_rows != 0 ? strip_rows : (config_.strip_rows != 0 ? config_.strip_rows : 128),
+                          strip_cols != 0 ? strip_cols : config_.strip_cols});
 }
 
 uint64_t Batch::Submit(const vqm_ss2_device_pair* pairs, uint32_t count) {
@@ -984,10 +981,12 @@ uint64_t Batch::Submit(const vqm_ss2_device_pair* pairs, uint32_t count) {
         for (const auto& [geometry, n] : per_geometry) {
             const auto [w, h] = geometry;
             const TuneChoice c = Tuner::Get().Choose(w, h, static_cast<PlaneFormat>(config_.plane_format), map_, n);
-            if (!pools_.HasPlan(w, h) && !pools_.HasShape(w, h)) pools_.SetStripShape(w, h, c.strip_rows, c.strip_cols);
+            const bool blocks = per_geometry.size() == 1 && config_.persistent == 0;
+            const TuneChoice::Launch& launch = blocks ? c.any : c.strips;
+            if (!pools_.HasPlan(w, h) && !pools_.HasShape(w, h)) pools_.SetStripShape(w, h, launch.shape);
             if (n > most) {
                 most = n;
-                chunks = c.chunks;
+                chunks = launch.chunks;
             }
         }
     }

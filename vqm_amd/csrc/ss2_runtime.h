@@ -173,9 +173,8 @@ public:
         return plans_.count(std::make_pair(width, height)) != 0;
     }
     // The strip shape of a geometry whose plan does not exist yet.
-    void SetStripShape(uint32_t width, uint32_t height, uint32_t strip_rows, uint32_t strip_cols,
-                       uint32_t row_parts = 1) {
-        shape_for_[std::make_pair(width, height)] = StripShape{strip_rows, strip_cols, row_parts};
+    void SetStripShape(uint32_t width, uint32_t height, const ScaleShape& shape) {
+        shape_for_[std::make_pair(width, height)] = shape;
     }
     bool HasShape(uint32_t width, uint32_t height) const {
         return shape_for_.count(std::make_pair(width, height)) != 0;
@@ -198,9 +197,6 @@ private:
             return std::tie(width, height, inputs) < std::tie(o.width, o.height, o.inputs);
         }
     };
-    struct StripShape {
-        uint32_t rows, cols, row_parts;
-    };
     struct Pool {
         std::vector<std::unique_ptr<Workspace>> idle;
         uint64_t each = 0;
@@ -211,7 +207,7 @@ private:
     uint64_t budget_;
     std::unique_ptr<Arena> arena_;
     std::map<std::pair<uint32_t, uint32_t>, std::unique_ptr<DevicePlan>> plans_;
-    std::map<std::pair<uint32_t, uint32_t>, StripShape> shape_for_;
+    std::map<std::pair<uint32_t, uint32_t>, ScaleShape> shape_for_;
     std::map<Key, Pool> pools_;
     uint64_t bytes_ = 0, peak_ = 0;
 };

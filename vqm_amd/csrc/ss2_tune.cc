@@ -50,50 +50,63 @@ TuneChoice Tuner::Choose(uint32_t width, uint32_t height, PlaneFormat format, Ma
     const uint8_t* src[2] = {inputs.as<uint8_t>(), inputs.as<uint8_t>() + image};
 
     TuneChoice best;
-    float best_per_pair = std::numeric_limits<float>::infinity();
-    for (uint32_t strip : kStripRows) {
-        for (uint32_t cols : kStripWidths) {
-            WorkspacePools pools(format, strip, cols, 0);
-            const DevicePlan& plan = pools.PlanFor(width, height);
-            const uint64_t each = pools.Need(width, height, false);
-            const uint32_t n =
-                static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(cls, kTuneBytes / each)));
-            Lane lane(n);
-            std::vector<std::unique_ptr<Workspace>> ws;
-            std::vector<LaunchEntry> entries(n);
-            for (uint32_t i = 0; i < n; ++i) {
-                ws.push_back(pools.Acquire(width, height, false));
-                entries[i].plan = &plan;
-                entries[i].ws = ws.back().get();
-                entries[i].src[0] = src[0];
-                entries[i].src[1] = src[1];
-            }
-            for (uint32_t chunks : kChunks) {
-                if (chunks > n) continue;
-                lane.Launch(format, map, ctx.lut, entries.data(), n, chunks);  // warm-up
+    constexpr float kInfinity = std::numeric_limits<float>::infinity();
+    float best_settable = kInfinity, best_any = kInfinity, best_strips = kInfinity;  // ms a pair
+    const std::vector<ScaleShape> shapes =
+        TuneShapes(width, height, format, cls, static_cast<uint32_t>(std::max(ctx.cus, 1)));
+    for (size_t k = 0; k < shapes.size(); ++k) {
+        const ScaleShape& shape = shapes[k];
+        const bool settable = k < kTuneSettable;
+        WorkspacePools pools(format, shape.rows, shape.cols, 0);
+        pools.SetStripShape(width, height, shape);
+        const DevicePlan& plan = pools.PlanFor(width, height);
+        const uint64_t each = pools.Need(width, height, false);
+        const uint32_t n = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(cls, kTuneBytes / each)));
+        Lane lane(n);
+        std::vector<std::unique_ptr<Workspace>> ws;
+        std::vector<LaunchEntry> entries(n);
+        for (uint32_t i = 0; i < n; ++i) {
+            ws.push_back(pools.Acquire(width, height, false));
+            entries[i].plan = &plan;
+            entries[i].ws = ws.back().get();
+            entries[i].src[0] = src[0];
+            entries[i].src[1] = src[1];
+        }
+        for (uint32_t chunks : kChunks) {
+            if (chunks > n) continue;
+            lane.Launch(format, map, ctx.lut, entries.data(), n, chunks);  // warm-up
+            lane.Wait();
+            float ms = kInfinity;
+            for (int r = 0; r < kRepeats; ++r) {
+                const auto t0 = std::chrono::steady_clock::now();
+                lane.Launch(format, map, ctx.lut, entries.data(), n, chunks);
                 lane.Wait();
-                float ms = std::numeric_limits<float>::infinity();
-                for (int r = 0; r < kRepeats; ++r) {
-                    const auto t0 = std::chrono::steady_clock::now();
-                    lane.Launch(format, map, ctx.lut, entries.data(), n, chunks);
-                    lane.Wait();
-                    const auto t1 = std::chrono::steady_clock::now();
-                    ms = std::min(ms, std::chrono::duration<float, std::milli>(t1 - t0).count());
-                }
-                const float per_pair = ms / static_cast<float>(n);
+                const auto t1 = std::chrono::steady_clock::now();
+                ms = std::min(ms, std::chrono::duration<float, std::milli>(t1 - t0).count());
+            }
+            const float per_pair = ms / static_cast<float>(n);
+            if (settable) {
                 ++best.candidates;
-                if (strip == 64 && cols == kDefaultStripCols && chunks == 1)
+                if (shape.rows == 64 && shape.cols == kDefaultStripCols && chunks == 1)
                     best.default_ms = per_pair * static_cast<float>(cls);
-                if (per_pair < best_per_pair) {
-                    best_per_pair = per_pair;
-                    best.strip_rows = strip;
-                    best.strip_cols = cols;
+                if (per_pair < best_settable) {
+                    best_settable = per_pair;
+                    best.strip_rows = shape.rows;
+                    best.strip_cols = shape.cols;
                     best.chunks = chunks;
                 }
             }
+            if (shape.row_parts != 0 && per_pair < best_strips) {
+                best_strips = per_pair;
+                best.strips = {shape, chunks};
+            }
+            if (per_pair < best_any) {
+                best_any = per_pair;
+                best.any = {shape, chunks};
+            }
         }
     }
-    best.ms_per_launch = best_per_pair * static_cast<float>(cls);
+    best.ms_per_launch = best_settable * static_cast<float>(cls);
     cache_[key] = best;
     return best;
 }
