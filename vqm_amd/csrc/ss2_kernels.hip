@@ -667,19 +667,57 @@ __device__ void stage_chroma(ConstAS<SourceDesc>* d, GlobalAS<const uint8_t>* sr
     }
 }
 
+// The weights of a tile's columns and rows (Rows of them), staged in LDS for the
+// filters of more than two taps. Formed for each pixel (24 sines a pixel for
+// Lanczos-3) a 4K 4:2:0 pair took 1,183 us with Lanczos-3 and 500 with
+// Catmull-Rom, now 503 and 344, a 1080p pair 367 and 176, now 184 and 135; and
+// the registers of the sums spilled six values of the four-row form, in all
+// formats (4K 8-bit bilinear 97.1 us of prepare, now 93.0).
+template <uint32_t Rows>
+struct ChromaWeights {
+    float x[kPrepTileW][kMaxTaps], y[Rows][kMaxTaps];
+};
+
+// Block-wide, as stage_chroma: thread `tid` forms every threads-th column or
+// row from pixel (x0, y0).
+template <uint32_t Rows>
+__device__ void stage_weights(ConstAS<SourceDesc>* d, uint32_t x0, uint32_t y0, uint32_t tid, uint32_t threads,
+                              ChromaWeights<Rows>& weights) {
+    for (uint32_t i = tid; i < kPrepTileW + Rows; i += threads) {
+        const bool column = i < kPrepTileW;
+        const uint32_t at = column ? i : i - kPrepTileW;
+        float w[kMaxTaps] = {};
+        int first;
+        axis_weights<false>(d->filter, (column ? x0 : y0) + at, column ? d->sub_w : d->sub_h,
+                            column ? d->shift_x : d->shift_y, w, &first);
+        float* const out = column ? weights.x[at] : weights.y[at];
+#pragma unroll
+        for (int j = 0; j < kMaxTaps; ++j) out[j] = w[j];
+    }
+}
+
 // Both chroma samples of pixel (x, y): the two chroma planes share their
 // size and siting, so one set of taps serves both. Rows are summed first,
 // then weighted by the vertical taps. With a staged window the samples come
 // from LDS (the same values, in the same order), else from the planes.
-// Bilinear: the descriptor's filter is 0.
+// Bilinear: the descriptor's filter is 0; else staged_x and staged_y are the
+// staged weights of x and y.
 template <bool Bilinear>
 __device__ __forceinline__ float2 chroma_samples(ConstAS<SourceDesc>* d, GlobalAS<const uint8_t>* src,
-                                                 const float2* window, const ChromaWindow& cw, uint32_t x,
-                                                 uint32_t y) {
+                                                 const float2* window, const ChromaWindow& cw, uint32_t x, uint32_t y,
+                                                 const float* staged_x, const float* staged_y) {
     float wx[Bilinear ? 2 : kMaxTaps], wy[Bilinear ? 2 : kMaxTaps];
-    int fx, fy;
-    const int tx = axis_weights<Bilinear>(d->filter, x, d->sub_w, d->shift_x, wx, &fx);
-    const int ty = axis_weights<Bilinear>(d->filter, y, d->sub_h, d->shift_y, wy, &fy);
+    int fx, fy, tx, ty;
+    if constexpr (Bilinear) {
+        tx = axis_weights<true>(0u, x, d->sub_w, d->shift_x, wx, &fx);
+        ty = axis_weights<true>(0u, y, d->sub_h, d->shift_y, wy, &fy);
+    } else {
+        tx = ty = tap_count(d->filter);
+        fx = static_cast<int>(first_tap(tx, chroma_pos(x, d->sub_w, d->shift_x)));
+        fy = static_cast<int>(first_tap(ty, chroma_pos(y, d->sub_h, d->shift_y)));
+#pragma unroll
+        for (int k = 0; k < kMaxTaps; ++k) wx[k] = staged_x[k], wy[k] = staged_y[k];
+    }
     float sum_u = 0.0f, sum_v = 0.0f;
     if (window != nullptr) {
         // The first taps are non-decreasing in x and y, so they lie within
@@ -747,8 +785,7 @@ __device__ __forceinline__ void plane4(ConstAS<SourceDesc>* d, GlobalAS<const ui
 // The columns of a lane's four pixels in the staged window, bilinear: the right
 // tap's weight (the left's is one less it) and the left tap's entry in a row.
 // They are the same in all four rows; formed again for each, a 1080p 8-bit
-// 4:2:0 pair prepared in 33.9 us, now 32.7. (The registers they take spill six
-// values around the loop over the rows, none within it.)
+// 4:2:0 pair prepared in 33.9 us, without that in 32.7.
 struct BilinearColumns {
     float t[4];
     uint32_t at[4];
@@ -797,9 +834,11 @@ __device__ __forceinline__ void bilinear4(ConstAS<SourceDesc>* d, const float2* 
 // rows ahead of the chroma gave nothing (and spilled), leaving out every stage
 // that these formats pass by 4 us of 123.
 // `window` is the tile's staged chroma, or null to read the chroma planes
-// directly.
+// directly; `weights` the staged ones of the tile from pixel (X0, Y0).
+template <uint32_t Rows>
 __device__ __forceinline__ void row4(ConstAS<SourceDesc>* d, GlobalAS<const uint8_t>* src, const float2* window,
-                                     const ChromaWindow& cw, const BilinearColumns& columns, uint32_t bx,
+                                     const ChromaWindow& cw, const BilinearColumns& columns,
+                                     const ChromaWeights<Rows>& weights, uint32_t X0, uint32_t Y0, uint32_t bx,
                                      const uint32_t (&col)[4], uint32_t y, uint32_t W, float (&lin)[4][3]) {
     float3 px[4];
     {
@@ -817,8 +856,9 @@ __device__ __forceinline__ void row4(ConstAS<SourceDesc>* d, GlobalAS<const uint
             for (int k = 0; k < 4; ++k) {
                 // One copy of the code, the pixels passing through it in turn.
                 const uint32_t x = k == 0 ? col[0] : k == 1 ? col[1] : k == 2 ? col[2] : col[3];
-                const float2 uv = d->filter == 0 ? chroma_samples<true>(d, src, window, cw, x, y)
-                                                 : chroma_samples<false>(d, src, window, cw, x, y);
+                const float2 uv =
+                    d->filter == 0 ? chroma_samples<true>(d, src, window, cw, x, y, nullptr, nullptr)
+                                   : chroma_samples<false>(d, src, window, cw, x, y, weights.x[x - X0], weights.y[y - Y0]);
                 const float3 p = make_float3(px[0].x, uv.x, uv.y);
                 px[0] = px[1];
                 px[1] = px[2];
@@ -1082,7 +1122,10 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
     ConstAS<SourceDesc>* sd = nullptr;
     const float2* window = nullptr;
     decode::ChromaWindow cw{0, 0, 0, 0};
+    decode::ChromaWeights<kPrepTileH>* weights = nullptr;
     if constexpr (General) {
+        __shared__ decode::ChromaWeights<kPrepTileH> staged;
+        weights = &staged;
         // Formats other than 8-bit sRGB RGB decode per pixel (block-uniform).
         const SourceDesc* sdp = image ? pdp->source[1] : pdp->source[0];
         if (sdp != nullptr && as_const(sdp)->kind != 0u) {
@@ -1092,11 +1135,14 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
             // in LDS once, instead of each pixel loading its taps from the
             // planes (8 loads a pixel for bilinear 4:2:0, 72 for Lanczos-3).
             __shared__ float2 chroma[decode::kChromaWindow];
-            if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0) &&
-                decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), tr.Y0,
-                                      min(tr.Y0 + kPrepTileH - 1u, H - 1u), &cw)) {
-                decode::stage_chroma(sd, src, cw, threadIdx.x, 64u * kPrepWaves<General>, chroma);
-                window = chroma;
+            if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0)) {
+                constexpr uint32_t kThreads = 64u * kPrepWaves<General>;
+                if (sd->filter != 0) decode::stage_weights(sd, X0, tr.Y0, threadIdx.x, kThreads, *weights);
+                if (decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), tr.Y0,
+                                          min(tr.Y0 + kPrepTileH - 1u, H - 1u), &cw)) {
+                    decode::stage_chroma(sd, src, cw, threadIdx.x, kThreads, chroma);
+                    window = chroma;
+                }
                 __syncthreads();
             }
         }
@@ -1133,7 +1179,7 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
         if constexpr (General) {
             if (!table) {
                 const uint32_t col[4] = {base_col(0), base_col(1), base_col(2), base_col(3)};
-                decode::row4(sd, src, window, cw, columns, bx, col, yc, W, lin);
+                decode::row4(sd, src, window, cw, columns, *weights, X0, tr.Y0, bx, col, yc, W, lin);
             }
         }
         if (table) {
@@ -1245,7 +1291,7 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
 // wave's chain of rows, take the split form below.)
 //
 // Registers: 92 in the reference form, 91 in the difference form (five waves
-// a SIMD), 128 in the general decode (four).
+// a SIMD), 127 in the general decode (four).
 template <typename Lay, bool General, bool Ref>
 __global__ __launch_bounds__(64 * kPrepWaves<General>) __attribute__((amdgpu_waves_per_eu(General ? 4 : 5))) void
 prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ work, uint32_t tiles,
@@ -1285,7 +1331,7 @@ prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ w
 // 41.2; U16 planes 24.5 against 24.9, 22.8 against 23.1, 37.9 against 36.3.
 // General decode, up to 4 tiles a CU: 512x512 8-bit 4:2:0 20.2 -> 10.9 us, 10-bit
 // PQ 23.3 -> 11.8, 1280x720 (920 tiles) 24.9 -> 21.0 and 31.6 -> 24.4; 1080p
-// (2,040) 33.7 against 36.6 and 42.0 against 41.2. 86 registers.
+// (2,040) 33.7 against 36.6 and 42.0 against 41.2. 82 registers.
 template <bool General> constexpr uint32_t kSplitTiles = (General ? 4 : 14) * 256;
 
 template <typename Lay, bool General, bool Ref>
@@ -1330,16 +1376,19 @@ __global__ __launch_bounds__(256) void prepare_split_kernel(const PairDesc* __re
             __shared__ float2 chroma[decode::kChromaWindow];
             const float2* window = nullptr;
             decode::ChromaWindow cw{0, 0, 0, 0};
-            if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0) &&
-                decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), Y0, min(Y0 + kWaveRows - 1u, H - 1u), &cw)) {
-                decode::stage_chroma(sd, src, cw, threadIdx.x, 256u, chroma);
-                window = chroma;
+            __shared__ decode::ChromaWeights<kWaveRows> weights;
+            if (sd->family == 2 && (sd->sub_w != 0 || sd->sub_h != 0)) {
+                if (sd->filter != 0) decode::stage_weights(sd, X0, Y0, threadIdx.x, 256u, weights);
+                if (decode::chroma_window(sd, X0, min(X0 + kPrepTileW - 1u, W - 1u), Y0, min(Y0 + kWaveRows - 1u, H - 1u), &cw)) {
+                    decode::stage_chroma(sd, src, cw, threadIdx.x, 256u, chroma);
+                    window = chroma;
+                }
                 __syncthreads();
             }
             const uint32_t col[4] = {base_col(0), base_col(1), base_col(2), base_col(3)};
             decode::BilinearColumns columns{};
             if (window != nullptr && sd->filter == 0) columns = decode::bilinear_columns(sd, cw, col);
-            decode::row4(sd, src, window, cw, columns, bx, col, yc, W, lin);
+            decode::row4(sd, src, window, cw, columns, weights, X0, Y0, bx, col, yc, W, lin);
         }
     }
     if (from_table) {
