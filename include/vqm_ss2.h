@@ -430,8 +430,8 @@ typedef struct vqm_ss2_batch_config {
                                 its stage times then report the whole graph
                                 as the prepare stage. 2: the same for
                                 submissions of up to 8 pairs (the Python
-                                binding's default). 0: eager, 3-7% faster on
-                                one to four 1080p pairs. */
+                                binding's default). 0: eager, 7-13% faster
+                                on one to eight pairs. */
 } vqm_ss2_batch_config;
 
 /* One pair of caller-owned device images (packed u8 sRGB RGB). */

@@ -830,9 +830,13 @@ __device__ __forceinline__ void bilinear4(ConstAS<SourceDesc>* d, const float2* 
 // four, so that its branches are taken and its descriptor fields read once
 // (a pixel at a time took 18 scalar loads and 123 scalar instructions each).
 // Prepare of one pair: 1080p 8-bit 4:2:0 49.7 -> 36.0 us, 4K 10-bit PQ 4:2:0
-// 170 -> 149 us. What bounds it now is VALU issue: loading the luma of all four
-// rows ahead of the chroma gave nothing (and spilled), leaving out every stage
-// that these formats pass by 4 us of 123.
+// 170 -> 149 us. What bounds it now is waiting with four waves a SIMD: they wait
+// in 53% of their cycles at 1080p (8-bit), whose 4,080 waves are all resident at
+// once, in 45% at 4K and 40% there in PQ, and issue 0.56, 0.80 and 0.85 vector
+// instructions a CU-cycle of 1.78; a wave makes some 130 scalar loads and 900
+// scalar instructions. Loading the luma of all four rows ahead of the chroma
+// gave nothing (and spilled), leaving out every stage that these formats pass by
+// 4 us of 123.
 // `window` is the tile's staged chroma, or null to read the chroma planes
 // directly; `weights` the staged ones of the tile from pixel (X0, Y0).
 template <uint32_t Rows>
@@ -1290,8 +1294,7 @@ __device__ __forceinline__ void prepare_tile(const TileRef& tr, uint32_t half, c
 // in the mixed form 0.90 -> 0.86 ms. (Launches of few tiles, whose time is one
 // wave's chain of rows, take the split form below.)
 //
-// Registers: 92 in the reference form, 91 in the difference form (five waves
-// a SIMD), 127 in the general decode (four).
+// Registers: 93 in the table decode's two forms (five waves a SIMD), 127 in the general decode (four).
 template <typename Lay, bool General, bool Ref>
 __global__ __launch_bounds__(64 * kPrepWaves<General>) __attribute__((amdgpu_waves_per_eu(General ? 4 : 5))) void
 prepare_kernel(const PairDesc* __restrict__ pairs, const WorkRef* __restrict__ work, uint32_t tiles,

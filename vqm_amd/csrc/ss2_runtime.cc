@@ -271,7 +271,7 @@ namespace {
 // The event that ends a stage. It rides on the stage's kernel, or is recorded
 // behind it: for launches split over two streams, and where images were
 // uploaded on the stream, whose next upload starts later behind a riding event
-// (6 pairs of 1080p from host memory over two pipelines: 1,606 us against
+// (6 pairs of 1080p from host memory over three pipelines: 1,606 us against
 // 1,555). The runtime keeps a riding event's kernel until its stream is
 // synchronized or copies again: a lane's next launch does, with its
 // descriptors; Pipeline::Finish sees to it for pairs.
